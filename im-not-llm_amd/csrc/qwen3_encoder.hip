@@ -42,6 +42,7 @@
 
 #include "../../include/inl_encoder.h"
 #include "inl_common.hpp"
+#include "skinny.hpp"
 
 struct inl_qwen3 {
   inl_qwen3_config cfg;
@@ -71,9 +72,22 @@ namespace {
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct Layout {
-  size_t ids, pos, cu, resid, x, a, b, sched, gemm, total;
+  size_t ids, pos, cu, resid, x, a, b, hf, xf, sched, gemm, total;
   int64_t a_w, b_w;  // row widths (elements) of the two activation buffers
 };
+
+int32_t longest_text(int32_t n_texts, const int32_t* cu) {
+  int32_t t = 0;
+  for (int b = 0; b < n_texts; ++b) t = std::max(t, cu[b + 1] - cu[b]);
+  return t;
+}
+
+// Whether a batch's layers run on the kernels for a few token rows (they take
+// P and V of the attention in f16, which INL_ATTN_PV_BF16 forbids).
+bool is_few(const inl_qwen3_config& c, int64_t n, int32_t longest) {
+  return c.attn_flags == 0 &&
+         few_fits(c.dtype, n, longest, c.hidden, c.heads, c.kv_heads, c.head_dim, c.intermediate);
+}
 
 int layout(const inl_qwen3* e, int32_t n_texts, const int32_t* cu, Layout* L) {
   const inl_qwen3_config& c = e->cfg;
@@ -91,6 +105,9 @@ int layout(const inl_qwen3* e, int32_t n_texts, const int32_t* cu, Layout* L) {
   L->x = take((size_t)n * c.hidden * es);
   L->a = take((size_t)n * L->a_w * es);
   L->b = take((size_t)n * L->b_w * es);
+  const bool few = is_few(c, n, longest_text(n_texts, cu));
+  L->hf = take(few ? few_h_bytes(n, c.hidden) : 0);
+  L->xf = take(few ? few_x_bytes(c.dtype, n, L->b_w) : 0);
   inl_attn_desc d{};
   d.n_texts = n_texts;
   d.cu_seqlens_host = cu;
@@ -327,6 +344,10 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
   char* A = ws + L.a;
   char* B = ws + L.b;
   void* gws = ws + L.gemm;
+  const int32_t longest = longest_text(n_texts, cu);
+  const bool few = is_few(c, n, longest);
+  char* hf = ws + L.hf;
+  char* xf = ws + L.xf;
   size_t gws_bytes = 0;
   rc = inl_linear_workspace_size(&gws_bytes);
   if (rc) return rc;
@@ -396,9 +417,29 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
   nr.round_tables = nr.round_norm = dt == INL_BF16;
 
   void* stream = sq;
-  int rc = inl_embed_fwd(n, d_ids, e->embed, c.vocab, c.hidden, dt, resid, c.hidden, stream);
+  int rc = few ? few_embed(dt, n, d_ids, e->embed, c.vocab, c.hidden, resid, hf, (hipStream_t)stream)
+               : inl_embed_fwd(n, d_ids, e->embed, c.vocab, c.hidden, dt, resid, c.hidden, stream);
   for (int i = 0; i < c.layers && !rc; ++i) {
     const inl_qwen3_layer_weights& w = e->layers[i];
+    if (few) {
+      hipStream_t sq = (hipStream_t)stream;
+      const SkinnyNext to_o = skinny_next(dt, w.o_proj, c.hidden, (int32_t)qd, false);
+      const SkinnyNext to_gu = skinny_next(dt, w.gate_up_proj, c.intermediate, c.hidden, true);
+      const SkinnyNext to_down = skinny_next(dt, w.down_proj, c.hidden, c.intermediate, false);
+      const SkinnyNext to_qkv = i + 1 < c.layers
+          ? skinny_next(dt, e->layers[i + 1].qkv_proj, (int32_t)qkv_w, c.hidden, false) : SkinnyNext{};
+      rc = skinny_launch(dt, n, (int32_t)qkv_w, c.hidden, hf, w.input_norm, c.eps, w.qkv_proj, SKINNY_STORE, A, L.a_w,
+                         nullptr, SkinnyNext{}, sq);
+      if (!rc) rc = few_attn(dt, n_texts, n, longest, d_cu, A, L.a_w, c.heads, c.kv_heads, w.q_norm, w.k_norm, c.eps,
+                             e->cos, e->sin, xf, to_o, sq);
+      if (!rc) rc = skinny_launch(dt, n, c.hidden, (int32_t)qd, xf, nullptr, 0.f, w.o_proj, SKINNY_ADD_F32, resid,
+                                  c.hidden, hf, to_gu, sq);
+      if (!rc) rc = skinny_launch(dt, n, c.intermediate, c.hidden, hf, w.post_attention_norm, c.eps, w.gate_up_proj,
+                                  SKINNY_SWIGLU, nullptr, 0, xf, to_down, sq);
+      if (!rc) rc = skinny_launch(dt, n, c.hidden, c.intermediate, xf, nullptr, 0.f, w.down_proj, SKINNY_ADD_F32,
+                                  resid, c.hidden, hf, to_qkv, sq);
+      continue;
+    }
     rc = inl_rms_norm_rows_fwd(n, c.hidden, resid, c.hidden, w.input_norm, dt, c.eps, dt, x, c.hidden, stream);
     if (!rc) rc = inl_linear_fwd(n, qkv_w, c.hidden, dt, x, c.hidden, w.qkv_proj, c.hidden, dt, A, L.a_w, 1.f, 0.f,
                                  gws, gws_bytes, stream);

@@ -1,0 +1,51 @@
+"""GPU Qwen3 encodes of few token rows (at most 128 in bf16, 64 in f32), which
+run on kernels of their own, against the numpy oracle (oracle/qwen3.py).
+
+Two layers of random weights at shapes that cover both hidden widths the path
+takes, one, two and four query heads per K/V head, and row counts at the edges
+of its 16-row blocks, of its text-length classes (32, 64, 128) and of the path
+itself. Tolerances are those of the general path's own test
+(tests/test_qwen3_e2e_gpu.py): f32 cosine 0.99999 and 2e-4 max-abs, bf16
+cosine 0.999 on the bf16-rounded weights."""
+import numpy as np
+import pytest
+
+from oracle import attention as oa
+from oracle import qwen3 as oq
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "0.6B": dict(),
+    "group1": dict(hidden=512, intermediate=2048, heads=8, kv_heads=8),
+    "group4": dict(intermediate=1024, heads=16, kv_heads=4),
+}
+CASES = [("0.6B", [1]), ("0.6B", [16]), ("0.6B", [17]), ("0.6B", [31, 1]), ("0.6B", [33]), ("0.6B", [5, 1, 32, 10]),
+         ("0.6B", [64]), ("0.6B", [65]), ("0.6B", [127]), ("0.6B", [3, 97, 28]), ("0.6B", [100, 29]),
+         ("group1", [23]), ("group1", [40, 24]), ("group4", [23]), ("group4", [64]), ("group4", [80])]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shape,lengths", CASES)
+def test_few_rows_against_oracle(shape, lengths, dtype, cuda, inl):
+    import torch
+    cfg = oq.Qwen3Config(vocab=512, layers=2, **SHAPES[shape])
+    w = oq.random_weights(cfg, seed=11)
+    td = torch.float32 if dtype == "f32" else torch.bfloat16
+    wd = {k: torch.from_numpy(np.ascontiguousarray(v)).to(cuda).to(td) for k, v in w.items()}
+    if dtype == "bf16":
+        w = {k: v.float().cpu().numpy() for k, v in wd.items()}
+    rng = np.random.default_rng(sum(lengths))
+    cu = oa.cu_from_lengths(lengths)
+    enc = inl.Qwen3Encoder(cfg, wd, max_positions=128)
+    print(f"case={shape} {dtype} {lengths}", flush=True)
+    for call in range(3):   # eager, captured and replayed
+        ids = rng.integers(0, cfg.vocab, sum(lengths))
+        got = enc.encode(ids, cu.tolist()).cpu().numpy().astype(np.float64)
+        ref = oq.encode(w, cfg, ids, cu)
+        cos = (got * ref).sum(1) / np.linalg.norm(got, axis=1) / np.linalg.norm(ref, axis=1)
+        if dtype == "f32":
+            assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4
+        else:
+            assert cos.min() >= 0.999
+    enc.close()
