@@ -21,6 +21,7 @@
 #include "../../include/inl_gdn.h"
 #include "attn_kernels.hpp"
 #include "inl_common.hpp"
+#include "gdn_chunk.hpp"
 #include "lanes.hpp"
 
 #pragma clang fp contract(off)
@@ -699,6 +700,8 @@ extern "C" int inl_gdn_rule_fwd(int64_t n_tokens, int32_t n_texts, const int32_t
   p.dk = key_dim;
   p.dv = value_dim;
   hipStream_t st = as_stream(stream);
+  const GdnChunkParams c{p.mixed, p.ms, g, beta, p.gs, out, p.os, p.cu, p.n, n_texts, p.nk, p.nv, p.dk, p.dv};
+  if (gdn_chunk_fits(c, dtype)) return gdn_chunk_launch(c, dtype, st);
   const dim3 grid((unsigned)value_heads, (unsigned)n_texts);
   if (dtype == INL_BF16) hipLaunchKernelGGL(gdn_rule_kernel<bf16>, grid, dim3(GDN_WAVES * 64), 0, st, p);
   else hipLaunchKernelGGL(gdn_rule_kernel<float>, grid, dim3(GDN_WAVES * 64), 0, st, p);

@@ -1,0 +1,626 @@
+// The gated delta rule in chunks, on the matrix cores (gfx950).
+//
+// The per-token recurrence (gdn.hip) is bound by vector FMAs and by its
+// serial chain: 0.59 us per token of the longest text at 16 heads, whatever
+// else the chip has to do. Over a chunk of C tokens the same recurrence is
+// (the reference's own chunked form, crates/inl-late/src/qwen3_5.rs:607-728):
+//
+//   A_ij = beta_i (k_i . k_j) e^(c_i - c_j), j < i        c = running sum of g
+//   T    = (I + A)^-1 diag(beta)
+//   R    = V - e^c K S          (rows scaled)             S: the state [dk, dv]
+//   U    = T R
+//   O    = e^c Q S + P U,       P_ij = (q_i . k_j) e^(c_i - c_j), j <= i
+//   S   <- e^(c_C) S + K^T (e^(c_C - c) U)
+//
+// Measured against the per-token kernel, rule alone, 16 heads, bf16: 16 texts
+// of 80 to 1,453 tokens 861 -> 264 us, 16 texts of 2,048 1,216 -> 510 us.
+//
+// Non-finite values: 0 times inf is NaN in a product, so an inf or NaN in a
+// token's row may reach earlier tokens of its own chunk and head as well.
+//
+// Two kernels. gdn_chunk_prep computes T and P of every chunk of every text
+// at once (one wave per chunk and head) and leaves them in the rows of `out`
+// that the chunk's results will replace: 2 C values of the row's 128, so no
+// workspace is needed. gdn_chunk_rule walks a text's chunks, one workgroup of
+// 8 waves per (text, head), wave w holding columns 16 w .. 16 w + 15 of S, U
+// and O in registers; only what all columns share (K, Q, K^T, T, P) is in LDS,
+// in operand order, so a chunk costs two barriers.
+//
+// Precision. State, R, U, T and P are f32 and enter the products as three
+// bf16 parts each (8 + 8 + 8 significand bits, rounded to nearest: the parts
+// add up to the f32 value), of whose nine products the six above 2^-27 are
+// summed in f32 by the MFMAs. bf16 K and Q are taken raw, as the one exact
+// part they are (three products), and their norms scale rows of the results.
+// The running sum of g is kept in f64, so that e^(c_i - c_j) is exact to f32
+// however far the sum has run. Against the f64 recurrence the error is no
+// larger than the per-token kernel's.
+//
+// An MFMA contraction of 32 takes its terms in any order that both operands
+// share. Here lane group g = lane / 16, element e = 4 h + r holds term 16 h +
+// 4 g + r: that is how a product's own registers lie (row 4 g + r of block h),
+// so S, R and U feed the next product without leaving their lane.
+#include "gdn_chunk.hpp"
+#include "attn_stream.hpp"
+#include "lanes.hpp"
+
+namespace inl {
+
+namespace {
+
+constexpr int GC_D = 128;     // key and value dim
+constexpr int GC_WAVES = 8;
+
+template <typename T>
+constexpr int gc_len() { return sizeof(T) == 2 ? 64 : 32; }   // f32: three parts of K, Q, K^T fit LDS at 32
+template <typename T>
+constexpr int gc_parts() { return sizeof(T) == 2 ? 1 : 3; }
+
+// Sum over the four lanes that share lane & 15, in all of them.
+__device__ __forceinline__ float gc_rows4(float x) {
+  float a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  a = b = a + b;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return a + b;
+}
+
+// x as N bf16 parts (N = 3: their sum is x to f32's last bit), two values per
+// conversion.
+template <int N>
+__device__ __forceinline__ void gc_split(const float (&x)[8], bf16x8 (&p)[N]) {
+  u32x4 w[N];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f32x2 r = {x[2 * j], x[2 * j + 1]};
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+      w[n][j] = u;
+      if (n + 1 < N) {
+        r[0] -= __builtin_bit_cast(float, u << 16);
+        r[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+      }
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < N; ++n) p[n] = __builtin_bit_cast(bf16x8, w[n]);
+}
+// hi + lo += a . b over 32 terms: the leading parts' product in hi, the smaller
+// ones in lo (their sum rounds at its own size), those below 2^-26 dropped.
+template <int NA, int NB>
+__device__ __forceinline__ void gc_mm(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x4& hi, f32x4& lo) {
+#pragma unroll
+  for (int s = 2; s > 0; --s)
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if (s - i >= 0 && s - i < NB) lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[s - i], lo, 0, 0, 0);
+  hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], hi, 0, 0, 0);
+}
+
+// Eight values of T as loaded, and as bf16 parts.
+template <typename T>
+struct Raw;
+template <>
+struct Raw<bf16> {
+  bf16x8 v;
+  __device__ __forceinline__ float squares() const {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += (float)v[e] * (float)v[e];
+    return s;
+  }
+  __device__ __forceinline__ void parts(bf16x8 (&p)[1]) const { p[0] = v; }
+};
+template <>
+struct Raw<float> {
+  float v[8];
+  __device__ __forceinline__ float squares() const {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += v[e] * v[e];
+    return s;
+  }
+  __device__ __forceinline__ void parts(bf16x8 (&p)[3]) const { gc_split<3>(v, p); }
+};
+// Loads at byte offset `off` of a buffer that starts at a chunk's first row and
+// ends with the text: rows past the end read as zeros, without a clamp or a
+// mask. The 8 terms of one operand and step: 4 at off, 4 at off + 16 terms.
+template <typename T>
+__device__ __forceinline__ void gc_load(Raw<T>& x, __amdgpu_buffer_rsrc_t r, uint32_t off) {
+  if constexpr (sizeof(T) == 2) {
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off + 32, 0, 0));
+    const u32x4 w = {a[0], a[1], b[0], b[1]};
+    x.v = __builtin_bit_cast(bf16x8, w);
+  } else {
+    const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    const f32x4 b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 64, 0, 0));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { x.v[e] = a[e]; x.v[4 + e] = b[e]; }
+  }
+}
+__device__ __forceinline__ float gc_load_f32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+
+// Clamped bounds of text b (a malformed table gives wrong rows, never an
+// access outside the tensors).
+__device__ __forceinline__ void gc_bounds(const int32_t* cu, int b, int64_t n, int64_t* begin, int64_t* end) {
+  const int64_t c0 = cu[b], c1 = cu[b + 1];
+  *begin = c0 < 0 ? 0 : (c0 > n ? n : c0);
+  *end = c1 < *begin ? *begin : (c1 > n ? n : c1);
+}
+
+// Inclusive sum over the wave's lanes, in f64.
+__device__ __forceinline__ double gc_scan(double x, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const double y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  return x;
+}
+
+// The buffers of the chunk at row t0: `rows` rows of a tensor of f32 or T.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gc_rows_of(const void* base, int64_t t0, int64_t stride,
+                                                              int rows, int64_t width, int esize) {
+  return pp_rsrc(static_cast<const char*>(base) + t0 * stride * esize,
+                 (uint32_t)(((rows - 1) * stride + width) * esize));
+}
+
+// One wave per (chunk, value head). The chunks of text b are numbered from
+// cu[b] / C + b on: a device-side numbering without a prefix sum, with at most
+// one unused number per text.
+//
+// The inverse is taken by 16 x 16 blocks: the four diagonal blocks by forward
+// substitution side by side (lane = 16 block + column, 120 FMAs each), then
+// X_rc = -D_r sum_k A_rk X_kc on the f32 MFMAs, whose D registers (rows 4 g +
+// r) are the next product's B operand. One column of 64 per lane, 2,016 FMAs
+// in a chain of 64 rows, made the kernel 60 us at 138 chunks x 16 heads; this
+// form takes 45.
+template <typename T>
+__global__ __launch_bounds__(256) void gdn_chunk_prep(GdnChunkParams p) {
+  constexpr int C = gc_len<T>(), RB = C / 16, NP = gc_parts<T>(), AS = C + 4;
+  __shared__ __attribute__((aligned(16))) float s_a[4][C][AS];
+  __shared__ __attribute__((aligned(16))) float s_d[4][RB][16][20];
+  __shared__ __attribute__((aligned(16))) float s_ki[4][C], s_beta[4][C], s_qi[4][C];
+  __shared__ __attribute__((aligned(16))) double s_cum[4][C];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i16 = lane & 15, g = lane >> 4;
+  const int h = blockIdx.y * 4 + wave;
+  if (h >= p.nv) return;   // no workgroup barrier below
+  int lo = 0, hi = p.n_texts - 1;   // the last text whose numbers start at or before this one
+  const int64_t slot = blockIdx.x;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    int64_t b0, b1;
+    gc_bounds(p.cu, mid, p.n, &b0, &b1);
+    if (b0 / C + mid <= slot) lo = mid;
+    else hi = mid - 1;
+  }
+  int64_t begin, end;
+  gc_bounds(p.cu, lo, p.n, &begin, &end);
+  const int64_t t0 = begin + (slot - begin / C - lo) * C;
+  if (t0 < begin || t0 >= end) return;
+  const int rows = (int)min((int64_t)C, end - t0);
+  const int kh = h / (p.nv / p.nk);
+  const int ES = (int)sizeof(T);
+  const int64_t width = (int64_t)2 * p.nk * GC_D + (int64_t)p.nv * GC_D;
+  const __amdgpu_buffer_rsrc_t mr = gc_rows_of(p.mixed, t0, p.ms, rows, width, ES);
+  const __amdgpu_buffer_rsrc_t gr = gc_rows_of(p.g, t0, p.gs, rows, p.nv, 4);
+  const __amdgpu_buffer_rsrc_t br = gc_rows_of(p.beta, t0, p.gs, rows, p.nv, 4);
+  const __amdgpu_buffer_rsrc_t orr = gc_rows_of(p.out, t0, p.os, rows, (int64_t)p.nv * GC_D, 4);
+  auto sync = [] __attribute__((always_inline)) () {   // this wave's LDS writes, read by its other lanes
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+
+  // 16 rows as operands; returns their sums of squares
+  auto load_rows = [&](int64_t off, int rb, bf16x8 (&f)[4][NP]) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)((16 * rb + i16) * p.ms + off + 4 * g) * ES;
+    Raw<T> x[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) gc_load<T>(x[s], mr, at + 32 * s * ES);
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      ss += x[s].squares();
+      x[s].parts(f[s]);
+    }
+    return gc_rows4(ss);
+  };
+  auto dot = [&](const bf16x8 (&a)[4][NP], const bf16x8 (&b)[4][NP]) __attribute__((always_inline)) {
+    f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) gc_mm<NP, NP>(a[s], b[s], hi, lo);
+    if constexpr (NP > 1) hi += lo;
+    return hi;
+  };
+  const int64_t q_off = (int64_t)kh * GC_D, k_off = (int64_t)(p.nk + kh) * GC_D;
+  const float gv = lane < C ? gc_load_f32(gr, (uint32_t)(lane * p.gs + h) * 4) : 0.f;
+  const float bv = lane < C ? gc_load_f32(br, (uint32_t)(lane * p.gs + h) * 4) : 0.f;
+  bf16x8 kf[RB][4][NP];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const float ss = load_rows(k_off, rb, kf[rb]);
+    if (lane < 16) s_ki[wave][16 * rb + lane] = 1.0f / sqrtf(ss + 1e-6f);
+  }
+  const double cum = gc_scan((double)gv, lane);
+  {
+    if (lane < C) {
+      s_cum[wave][lane] = cum;
+      s_beta[wave][lane] = bv;
+    }
+  }
+  const float dk_scale = 1.0f / sqrtf((float)GC_D);
+  auto put = [&](int i, int c, float v) __attribute__((always_inline)) {   // rows past the end are dropped
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), orr,
+                                          (uint32_t)(i * p.os + (int64_t)h * GC_D + c) * 4, 0, 0);
+  };
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    bf16x8 qf[4][NP];
+    const float qs = load_rows(q_off, rb, qf);
+    if (lane < 16) s_qi[wave][16 * rb + lane] = dk_scale / sqrtf(qs + 1e-6f);
+    sync();
+    const f32x4 ki = *reinterpret_cast<const f32x4*>(&s_ki[wave][16 * rb + 4 * g]);
+    const f32x4 bi = *reinterpret_cast<const f32x4*>(&s_beta[wave][16 * rb + 4 * g]);
+    const f32x4 qi = *reinterpret_cast<const f32x4*>(&s_qi[wave][16 * rb + 4 * g]);
+    double ci[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ci[r] = s_cum[wave][16 * rb + 4 * g + r];
+#pragma unroll
+    for (int cb = 0; cb <= rb; ++cb) {
+      const f32x4 kk = dot(kf[rb], kf[cb]), qk = dot(qf, kf[cb]);
+      const int j = 16 * cb + i16;
+      const float kj = s_ki[wave][j];
+      const double cj = s_cum[wave][j];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * rb + 4 * g + r;
+        const float dec = i >= j ? expf((float)(ci[r] - cj)) * kj : 0.f;
+        s_a[wave][i][j] = kk[r] * ki[r] * dec * bi[r];
+        put(i, 64 + j, i >= j ? qk[r] * qi[r] * dec : 0.f);
+      }
+    }
+    if (rb % 2 == 0)   // the other half of the operand's 32 columns
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        put(16 * rb + 4 * g + r, 64 + 16 * (rb + 1) + i16, 0.f);
+        put(16 * rb + 4 * g + r, 16 * (rb + 1) + i16, 0.f);
+      }
+  }
+  sync();
+  if (lane < rows) {
+    // The chunk's row scales, in columns of T that no operand reads (those of
+    // rows 0 .. 31 past the first step): token t in row t % 32.
+    const double all = s_cum[wave][rows - 1];
+    const float ec = expf((float)cum);
+    const int c = 32 + 4 * (lane >> 5);
+    put(lane & 31, c, ec * s_ki[wave][lane]);
+    put(lane & 31, c + 1, ec * s_qi[wave][lane]);
+    put(lane & 31, c + 2, expf((float)(all - cum)) * s_ki[wave][lane]);
+    if (lane == 0) put(0, 35, expf((float)all));
+  }
+  {   // diagonal blocks: lane holds column i16 of block g
+    const int blk = g < RB ? g : 0;
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+      for (int k = 0; k < i; k += 4) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(&s_a[wave][16 * blk + i][16 * blk + k]);
+        s0 = __builtin_fmaf(a[0], x[k], s0);
+        if (k + 1 < i) s1 = __builtin_fmaf(a[1], x[k + 1], s1);
+        if (k + 2 < i) s0 = __builtin_fmaf(a[2], x[k + 2], s0);
+        if (k + 3 < i) s1 = __builtin_fmaf(a[3], x[k + 3], s1);
+      }
+      x[i] = i16 == i ? 1.0f : -(s0 + s1);
+      if (g < RB) s_d[wave][blk][i][i16] = x[i];
+    }
+  }
+  sync();
+  f32x4 X[RB][RB];   // X[rb][cb]: rows 16 rb + 4 g + r, column 16 cb + i16
+  auto mm16 = [&](const f32x4& a, const f32x4& b, f32x4 acc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], acc, 0, 0, 0);
+    return acc;
+  };
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const f32x4 d = *reinterpret_cast<const f32x4*>(&s_d[wave][rb][i16][4 * g]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) X[rb][rb][r] = s_d[wave][rb][4 * g + r][i16];
+#pragma unroll
+    for (int cb = 0; cb < rb; ++cb) {
+      f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = cb; kb < rb; ++kb)
+        y = mm16(*reinterpret_cast<const f32x4*>(&s_a[wave][16 * rb + i16][16 * kb + 4 * g]), X[kb][cb], y);
+      X[rb][cb] = -mm16(d, y, (f32x4){0.f, 0.f, 0.f, 0.f});
+    }
+#pragma unroll
+    for (int cb = 0; cb <= rb; ++cb) {
+      const float bj = s_beta[wave][16 * cb + i16];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) put(16 * rb + 4 * g + r, 16 * cb + i16, X[rb][cb][r] * bj);
+    }
+  }
+}
+
+// LDS of gdn_chunk_rule: fragments of 1 KiB (16 bytes per lane).
+template <typename T>
+struct GcLds {
+  static constexpr int C = gc_len<T>(), RB = C / 16, TS = C / 32, NP = gc_parts<T>();
+  static constexpr int KF = 0;                        // [RB][4][NP]
+  static constexpr int QF = KF + RB * 4 * NP * 1024;
+  static constexpr int KT = QF + RB * 4 * NP * 1024;  // [8][TS][NP]
+  static constexpr int TF = KT + 8 * TS * NP * 1024;  // [RB][TS][3]
+  static constexpr int PF = TF + RB * TS * 3 * 1024;
+  static constexpr int VEC = PF + RB * TS * 3 * 1024; // row scales [3][C] f32, e^(c_C)
+  static constexpr int TOTAL = VEC + 3 * C * 4 + 16;
+};
+
+template <typename T>
+__global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p) {
+  using L = GcLds<T>;
+  constexpr int C = L::C, RB = L::RB, TS = L::TS, NP = L::NP;
+  constexpr int FK = RB * 4 / GC_WAVES;   // K (and Q) fragments a wave stages
+  constexpr int FT = 8 * TS / GC_WAVES;   // K^T fragments
+  constexpr int FP = RB * TS;             // T (and P) fragments in all: wave w stages fragment w
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int h = blockIdx.x, b = blockIdx.y;
+  int64_t begin, end;
+  gc_bounds(p.cu, b, p.n, &begin, &end);
+  if (end <= begin) return;
+  const int kh = h / (p.nv / p.nk);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i16 = lane & 15, g = lane >> 4;
+  const int ES = (int)sizeof(T);
+  const int64_t width = (int64_t)2 * p.nk * GC_D + (int64_t)p.nv * GC_D;
+  const uint32_t q_off = (uint32_t)kh * GC_D, k_off = (uint32_t)(p.nk + kh) * GC_D;
+  const uint32_t v_off = (uint32_t)2 * p.nk * GC_D + (uint32_t)h * GC_D + 16 * wave + i16;
+  const uint32_t ms = (uint32_t)p.ms, os = (uint32_t)p.os;
+  auto frag = [&](int base, int i) __attribute__((always_inline)) {
+    return reinterpret_cast<bf16x8*>(smem + base + i * 1024 + lane * 16);
+  };
+
+  // registers of the chunk to come
+  Raw<T> rk[FK], rq[FK], rt[FT];
+  float rT[8], rP[8], rs[4];
+  T rv[RB][4];
+  auto load_t = [&](__amdgpu_buffer_rsrc_t r, uint32_t off) __attribute__((always_inline)) {
+    if constexpr (sizeof(T) == 2)
+      return __builtin_bit_cast(bf16, (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+    else return gc_load_f32(r, off);
+  };
+  auto fetch = [&](int64_t t0) __attribute__((always_inline)) {
+    const int rows = (int)min((int64_t)C, end - t0);
+    const __amdgpu_buffer_rsrc_t mr = gc_rows_of(p.mixed, t0, p.ms, rows, width, ES);
+    const __amdgpu_buffer_rsrc_t orr = gc_rows_of(p.out, t0, p.os, rows, (int64_t)p.nv * GC_D, 4);
+#pragma unroll
+    for (int f = 0; f < FK; ++f) {
+      const int id = wave * FK + f, rb = id >> 2, s = id & 3;
+      const uint32_t at = (16 * rb + i16) * ms + 32 * s + 4 * g;
+      gc_load<T>(rk[f], mr, (at + k_off) * ES);
+      gc_load<T>(rq[f], mr, (at + q_off) * ES);
+    }
+#pragma unroll
+    for (int f = 0; f < FT; ++f) {
+      const int id = wave * FT + f, db = id / TS, ts = id % TS;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        rt[f].v[e] = load_t(mr, ((32 * ts + 16 * (e >> 2) + 4 * g + (e & 3)) * ms + k_off + 16 * db + i16) * ES);
+    }
+    {
+      const int id = wave < FP ? wave : 0, rb = id / TS, ts = id % TS;
+      const uint32_t at = ((16 * rb + i16) * os + (uint32_t)h * GC_D + 32 * ts + 4 * g) * 4;
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(orr, at + 64 * hh, 0, 0));
+        const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(orr, at + 256 + 64 * hh, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { rT[4 * hh + e] = a[e]; rP[4 * hh + e] = q[e]; }
+      }
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rv[rb][r] = load_t(mr, ((16 * rb + 4 * g + r) * ms + v_off) * ES);
+    if (wave == GC_WAVES - 1) {   // row scales, one token per lane
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        rs[n] = gc_load_f32(orr, ((lane & 31) * os + (uint32_t)h * GC_D + 32 + 4 * (lane >> 5) + n) * 4);
+    }
+  };
+
+  f32x4 S[8];   // rows 16 b + 4 g + r of column 16 wave + i16
+#pragma unroll
+  for (int i = 0; i < 8; ++i) S[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float* vec = reinterpret_cast<float*>(smem + L::VEC);
+
+  // The two waves of a SIMD leave each barrier together; with equal priority
+  // both split (VALU), then both multiply. Favouring one lets it run ahead into
+  // its MFMAs while the other splits.
+  if (wave < GC_WAVES / 2) __builtin_amdgcn_s_setprio(2);
+  fetch(begin);
+  for (int64_t t0 = begin; t0 < end; t0 += C) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the last chunk's readers are done
+    {
+#pragma unroll
+      for (int f = 0; f < FK; ++f) {
+        bf16x8 a[NP], q[NP];
+        rk[f].parts(a);
+        rq[f].parts(q);
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+          *frag(L::KF, (wave * FK + f) * NP + n) = a[n];
+          *frag(L::QF, (wave * FK + f) * NP + n) = q[n];
+        }
+      }
+#pragma unroll
+      for (int f = 0; f < FT; ++f) {
+        bf16x8 a[NP];
+        rt[f].parts(a);
+#pragma unroll
+        for (int n = 0; n < NP; ++n) *frag(L::KT, (wave * FT + f) * NP + n) = a[n];
+      }
+      if (wave < FP) {
+        bf16x8 a[3], q[3];
+        gc_split<3>(rT, a);
+        gc_split<3>(rP, q);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          *frag(L::TF, wave * 3 + n) = a[n];
+          *frag(L::PF, wave * 3 + n) = q[n];
+        }
+      }
+      if (wave == GC_WAVES - 1) {
+        if (lane < C) {
+#pragma unroll
+          for (int n = 0; n < 3; ++n) vec[n * C + lane] = t0 + lane < end ? rs[n] : 0.f;
+        }
+        if (lane == 0) vec[3 * C] = rs[3];
+      }
+    }
+    f32x4 v[RB], o[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[rb][r] = (float)rv[rb][r];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (t0 + C < end) fetch(t0 + C);
+
+    const float eall = vec[3 * C];
+    auto scale = [&](int which, int rb) __attribute__((always_inline)) {
+      return *reinterpret_cast<const f32x4*>(vec + which * C + 16 * rb + 4 * g);
+    };
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+    {   // R = V - e^c K S, O = e^c Q S
+      bf16x8 sp[4][3];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = S[2 * s + (e >> 2)][e & 3];
+        gc_split<3>(x, sp[s]);
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        f32x4 kh_ = zero, kl = zero, qh = zero, ql = zero;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          bf16x8 a[NP], q[NP];
+#pragma unroll
+          for (int n = 0; n < NP; ++n) {
+            a[n] = *frag(L::KF, (rb * 4 + s) * NP + n);
+            q[n] = *frag(L::QF, (rb * 4 + s) * NP + n);
+          }
+          gc_mm<NP, 3>(a, sp[s], kh_, kl);
+          gc_mm<NP, 3>(q, sp[s], qh, ql);
+        }
+        v[rb] -= scale(0, rb) * (kh_ + kl);
+        o[rb] = scale(1, rb) * (qh + ql);
+      }
+    }
+    bf16x8 up[TS][3];
+    auto split_rows = [&](const f32x4 (&m)[RB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int ts = 0; ts < TS; ++ts) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = m[2 * ts + (e >> 2)][e & 3];
+        gc_split<3>(x, up[ts]);
+      }
+    };
+    split_rows(v);   // R
+    // U = T R and O += P U: block row rb of the lower triangles ends in step rb / 2
+    auto lower = [&](int base, f32x4 (&m)[RB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        f32x4 lo = zero;
+#pragma unroll
+        for (int ts = 0; ts <= rb / 2; ++ts) {
+          bf16x8 a[3];
+#pragma unroll
+          for (int n = 0; n < 3; ++n) a[n] = *frag(base, (rb * TS + ts) * 3 + n);
+          gc_mm<3, 3>(a, up[ts], m[rb], lo);
+        }
+        m[rb] += lo;
+      }
+    };
+    f32x4 u[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) u[rb] = zero;
+    lower(L::TF, u);
+    split_rows(u);
+    lower(L::PF, o);
+    {
+      const int rows = (int)min((int64_t)C, end - t0);
+      const __amdgpu_buffer_rsrc_t orr = gc_rows_of(p.out, t0, p.os, rows, (int64_t)p.nv * GC_D, 4);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = o[rb][r];
+          __builtin_amdgcn_raw_buffer_store_b32(
+              __builtin_bit_cast(uint32_t, x), orr,
+              ((16 * rb + 4 * g + r) * os + (uint32_t)h * GC_D + 16 * wave + i16) * 4, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) u[rb] *= scale(2, rb);
+    split_rows(u);
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      f32x4 lo = zero;
+      S[db] *= eall;
+#pragma unroll
+      for (int ts = 0; ts < TS; ++ts) {
+        bf16x8 a[NP];
+#pragma unroll
+        for (int n = 0; n < NP; ++n) a[n] = *frag(L::KT, (db * TS + ts) * NP + n);
+        gc_mm<NP, 3>(a, up[ts], S[db], lo);
+      }
+      S[db] += lo;
+    }
+  }
+}
+
+template <typename T>
+int gdn_chunk_go(const GdnChunkParams& p, hipStream_t st) {
+  constexpr int C = gc_len<T>();
+  const int64_t slots = p.n / C + p.n_texts;
+  if (slots > 0x7fffffff) return fail(INL_E_UNSUPPORTED, "gdn_rule: too many tokens");
+  const int rc = set_max_dynamic_lds(reinterpret_cast<const void*>(&gdn_chunk_rule<T>), GcLds<T>::TOTAL);
+  if (rc) return rc;
+  hipLaunchKernelGGL(gdn_chunk_prep<T>, dim3((unsigned)slots, (unsigned)((p.nv + 3) / 4)), dim3(256), 0, st, p);
+  INL_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL(gdn_chunk_rule<T>, dim3((unsigned)p.nv, (unsigned)p.n_texts), dim3(64 * GC_WAVES),
+                     GcLds<T>::TOTAL, st, p);
+  INL_HIP_TRY(hipGetLastError());
+  return INL_OK;
+}
+
+}  // namespace
+
+bool gdn_chunk_fits(const GdnChunkParams& p, int32_t dtype) {
+  // both dims 128 (a row of `out` holds 2 x 64 values of T and P), rows that
+  // take the vector loads
+  const int64_t esize = dtype_size(dtype);
+  return p.dk == GC_D && p.dv == GC_D && p.ms % 4 == 0 && ((uintptr_t)p.mixed % (4 * esize)) == 0 && p.os % 4 == 0 &&
+         ((uintptr_t)p.out & 15) == 0 && p.ms <= (1 << 22) && p.os <= (1 << 22) && p.gs <= (1 << 22) &&   // a chunk's offsets fit 32 bits
+         (p.nv + 3) / 4 <= 65535 &&
+         // Short texts leave most of a chunk empty and still pay two launches:
+         // one text of 32 tokens took 23 us here and 21 per token, one of 64
+         // 25 and 39, 128 texts of 40 121 and 201. The lengths are on the
+         // device, so the line is drawn at their mean.
+         p.n >= 40 * (int64_t)p.n_texts;
+}
+
+int gdn_chunk_launch(const GdnChunkParams& p, int32_t dtype, hipStream_t st) {
+  return dtype == INL_BF16 ? gdn_chunk_go<bf16>(p, st) : gdn_chunk_go<float>(p, st);
+}
+
+}  // namespace inl

@@ -255,3 +255,37 @@ def test_tiny_late_tower_on_gpu_matches_golden(task, cuda, inl):
         worst = max(np.abs(a - np.asarray(r)).max() for a, r in zip(out, case[key]) if a.size)
         print(f"tiny late {task} {key}: {worst:.3g}", flush=True)
         assert worst < 1e-4
+
+
+# The chunked rule (key and value dim 128, 40 tokens a text on average): text
+# lengths at the edges of its 64-token (bf16) and 32-token (f32) chunks, empty
+# texts, texts that start off a chunk's multiple, head counts that do not fill
+# its workgroups of four, and gates from no decay to e^-30 (whose running sum
+# must not lose the small decays that follow). Against the f64 recurrence on
+# the same inputs: values are sums of order 1 over f32 products, so 2^-24 per
+# rounding, some 40 roundings deep: 5e-6 of the largest value.
+CHUNK_CASES = [
+    ("bf16", 2, 2, [64], "small"), ("bf16", 2, 2, [65, 63, 128], "small"), ("f32", 2, 2, [32, 33, 95], "small"),
+    ("f32", 1, 3, [97, 0, 31, 160], "mixed"), ("bf16", 1, 5, [1, 0, 200, 130, 0], "mixed"),
+    ("bf16", 2, 4, [257, 1, 1, 64, 129], "zero"), ("f32", 2, 4, [257, 1, 64], "zero"),
+]
+
+
+@pytest.mark.parametrize("case", CHUNK_CASES, ids=[f"{c[0]}-{c[1]}x{c[2]}-{c[4]}-{sum(c[3])}" for c in CHUNK_CASES])
+def test_chunked_rule_matches_recurrence(case, cuda, inl):
+    import torch
+    dtype, nk, nv, lens, gates = case
+    print(f"case=gdn_chunked_rule {case}", flush=True)
+    rng = np.random.default_rng(sum(lens))
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n, dk = int(cu[-1]), 128
+    mixed = og._r(rng.standard_normal((n, (2 * nk + nv) * dk)).astype(np.float32), dtype)
+    u = rng.uniform(0, 1, (n, nv))
+    g = {"small": -0.2 * u, "mixed": -np.where(u < 0.1, 30.0, 0.02 * u), "zero": 0 * u}[gates].astype(np.float32)
+    beta = rng.uniform(0, 1, (n, nv)).astype(np.float32)
+    got = inl.gdn_rule(_t(torch, mixed, cuda, _tdtype(torch, dtype)), cu.tolist(), nk, nv, dk, dk,
+                       _t(torch, g, cuda, torch.float32), _t(torch, beta, cuda, torch.float32)).cpu().numpy()
+    ref = og.rule_packed(mixed, cu, nk, nv, dk, dk, g.astype(np.float64), beta.astype(np.float64))
+    err = np.abs(got - ref).max() / np.abs(ref).max()
+    print(f"chunked rule: max error {err:.3g} of the largest value", flush=True)
+    assert err <= 5e-6
