@@ -10,16 +10,17 @@
 // synchronised: a call is one kernel launch, so the same call works under
 // graph capture and for every token count M.
 //
-// Kernel: 256 x 256 output tiles, 8 waves (two per SIMD) as 2 (w rows, i.e.
-// output columns) x 4 (x rows), each wave 128 x 64 = 4 x 2 blocks of
-// v_mfma_f32_32x32x16_bf16 (the w block is the MFMA's row operand, the x
-// block its column operand, so a lane's accumulator holds one output row and
-// four runs of four consecutive output columns). The K
-// loop runs through a 3-stage LDS ring of 32-wide k slices (32 KiB a stage),
-// filled by direct global -> LDS loads three stages ahead; each stage's MFMA
-// operands are read into registers one stage ahead. The workgroup is
-// persistent: its tiles form one stream of stages, so the next tile's first
-// loads are in flight while the current tile's epilogue stores run. The
+// Kernel, in its largest shape (four are built, see GemmShape): 256 x 256
+// output tiles, 8 waves (two per SIMD) as 2 (w rows, i.e. output columns) x 4
+// (x rows), each wave 128 x 64 = 4 x 2 blocks of v_mfma_f32_32x32x16_bf16 (the
+// w block is the MFMA's row operand, the x block its column operand, so a
+// lane's accumulator holds one output row and four runs of four consecutive
+// output columns). The K loop runs through an LDS ring of 32-wide k slices (3
+// stages of 32 KiB), filled by direct global -> LDS loads that many stages
+// ahead; each stage's MFMA operands are read into registers one stage ahead.
+// The workgroup is persistent: its tiles form one stream of stages, so the
+// next tile's first loads are in flight while the current tile's epilogue
+// stores run. The
 // epilogue goes through 4 KiB of LDS per wave, 32 rows x 128 bytes at a
 // time, so that every store instruction writes eight whole 128-byte row
 // segments (stores straight from the accumulator layout write 32-byte pieces
@@ -52,42 +53,42 @@ namespace inl {
 
 namespace {
 
-constexpr int GM_BN = 256;    // w rows (output columns) per tile: 2 waves x 128
 constexpr int GM_BK = 32;     // k per LDS stage (64-byte rows)
 constexpr int GM_ROW = GM_BK * 2;
-constexpr int GM_W = GM_BN * GM_ROW;            // 16 KiB of w rows per stage
 constexpr int GM_STG = 4096;                    // per-wave epilogue staging: 32 rows x 128 bytes
 constexpr int GM_XCDS = 8;
 
-// Kernel shape: NW waves as 2 (w rows) x NW / 2 (x rows), each 128 x 64;
-// an LDS ring of STAGES k slices; WPC workgroups per CU.
-template <int NW_, int STAGES_, int WPC_>
+// Kernel shape: NWN waves along the w rows x NWM along the x rows, each WNB x
+// WMB blocks of 32 x 32; an LDS ring of STAGES k slices; WPC workgroups per CU.
+template <int NWN_, int NWM_, int WNB_, int WMB_, int STAGES_, int WPC_>
 struct GemmShape {
-  static constexpr int NW = NW_;
-  static constexpr int WMW = NW / 2;                // waves along x
-  static constexpr int BM = WMW * 64;               // x rows (output rows) per tile
+  static constexpr int NWN = NWN_, NWM = NWM_, WNB = WNB_, WMB = WMB_;
+  static constexpr int NW = NWN * NWM;
+  static constexpr int BN = NWN * WNB * 32;         // w rows (output columns) per tile
+  static constexpr int BM = NWM * WMB * 32;         // x rows (output rows) per tile
   static constexpr int STAGES = STAGES_;
   static constexpr int WPC = WPC_;
+  static constexpr int W = BN * GM_ROW;
   static constexpr int X = BM * GM_ROW;
-  static constexpr int STAGE = GM_W + X;
+  static constexpr int STAGE = W + X;
   static constexpr int BLOCKS = STAGE / 1024;       // 1 KiB direct-load blocks per stage
   static constexpr int PER_WAVE = BLOCKS / NW;
-  static constexpr int W_PER_WAVE = GM_W / 1024 / NW;
+  static constexpr int W_PER_WAVE = W / 1024 / NW;
   static constexpr int RING = STAGES * STAGE;
   static constexpr int LDS = RING + NW * GM_STG;
-  static_assert(BLOCKS % NW == 0 && (GM_W / 1024) % NW == 0, "the direct loads split evenly over the waves");
+  static_assert(BLOCKS % NW == 0 && (W / 1024) % NW == 0, "the direct loads split evenly over the waves");
   static_assert(NW % 2 == 0, "w blocks of one wave share its parity (GEGLU)");
   static_assert(STAGES >= 2 && (STAGES - 1) * PER_WAVE <= 63, "vmcnt range");
 };
-// Shape 0: 8 waves, 256 x 256 tiles, 3 stages, one workgroup per CU (128 KiB
-// LDS). Shape 1: 4 waves, 128 x 256 tiles, 2 stages, two workgroups per CU
-// (64 KiB each), so that one workgroup computes while the other drains its
-// tile's stores. Outputs of at most 256 columns (one n-tile per 256 rows of
-// x, whose rows then stream from HBM with no reuse) run on shape 1: at
-// 139,124 rows 7-8 % faster than shape 0, whose 544 tiles make 2.1 rounds
-// over 256 CUs; wider outputs run on shape 0 (shape 1 was 4-15 % slower).
+// Four shapes. 0: 256 x 256 tiles, 8 waves, one workgroup per CU: the most
+// products per byte, and the least overlap of a tile's stores with anything.
+// 1: 256 (w) x 128, 4 waves, and 2: 128 x 128, 4 waves, two per CU: one
+// computes while the other drains its tile. 3: 64 x 64, 4 waves: short tiles
+// for outputs that would otherwise leave most of the chip idle.
 template <int SH>
-using GemmShapeOf = std::conditional_t<SH == 1, GemmShape<4, 2, 2>, GemmShape<8, 3, 1>>;
+using GemmShapeOf = std::conditional_t<SH == 0, GemmShape<2, 4, 4, 2, 3, 1>,
+                    std::conditional_t<SH == 1, GemmShape<2, 2, 4, 2, 2, 2>,
+                    std::conditional_t<SH == 2, GemmShape<2, 2, 2, 2, 4, 2>, GemmShape<2, 2, 1, 1, 6, 2>>>>;
 
 enum GemmEpi { EPI_PLAIN = 0, EPI_GEGLU = 1, EPI_GELU_MUL = 2 };
 
@@ -126,9 +127,10 @@ __device__ __forceinline__ float gelu_tanh(float v) {
 template <int SH, int EPI, bool OUT_BF16, bool ACC>
 __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) void gemm_bf16_kernel(GemmParams p) {
   using C = GemmShapeOf<SH>;
-  constexpr int GM_NW = C::NW, GM_BM = C::BM, GM_STAGES = C::STAGES, GM_STAGE = C::STAGE;
+  constexpr int GM_NW = C::NW, GM_BM = C::BM, GM_BN = C::BN, GM_W = C::W, GM_STAGES = C::STAGES, GM_STAGE = C::STAGE;
   constexpr int GM_PER_WAVE = C::PER_WAVE, GM_RING = C::RING;
-  // output columns per tile: a GEGLU tile's 256 w rows are 128 gate + 128 up
+  constexpr int WNB = C::WNB, WMB = C::WMB;
+  // output columns per tile: half of a GEGLU tile's w rows are gates, half up
   constexpr int BNO = EPI == EPI_GEGLU ? GM_BN / 2 : GM_BN;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int xcd = blockIdx.x % GM_XCDS;
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wn = wave / C::WMW, wm = wave % C::WMW;
+  const int wn = wave / C::NWM, wm = wave % C::NWM;
   const int l32 = lane & 31, hf = lane >> 5;
 
   // per-lane offsets of this wave's direct-load blocks inside a tile: blocks
@@ -215,40 +217,40 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
     }
   };
 
-  // fragment addresses (stage 0): w rows wn*128 + a*32 + l32, x rows wm*64 + b*32 + l32
-  uint32_t fa[4][2], fb[2][2];
+  // fragment addresses (stage 0): w rows (wn*WNB + a)*32 + l32, x rows (wm*WMB + b)*32 + l32
+  uint32_t fa[WNB][2], fb[WMB][2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) fa[a][ks] = opaque(lds0 + gm_swz(wn * 128 + a * 32 + l32, 2 * ks + hf));
+    for (int a = 0; a < WNB; ++a) fa[a][ks] = opaque(lds0 + gm_swz((wn * WNB + a) * 32 + l32, 2 * ks + hf));
 #pragma unroll
-    for (int b = 0; b < 2; ++b) fb[b][ks] = opaque(lds0 + GM_W + gm_swz(wm * 64 + b * 32 + l32, 2 * ks + hf));
+    for (int b = 0; b < WMB; ++b) fb[b][ks] = opaque(lds0 + GM_W + gm_swz((wm * WMB + b) * 32 + l32, 2 * ks + hf));
   }
 
-  f32x16 acc[4][2];
+  f32x16 acc[WNB][WMB];
   const f32x16 zero = {};
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < WNB; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = zero;
+    for (int b = 0; b < WMB; ++b) acc[a][b] = zero;
 
-  // MFMA operands of one 16-wide k step: 4 w blocks and 2 x blocks
+  // MFMA operands of one 16-wide k step: WNB w blocks and WMB x blocks
   struct Half {
-    u32x4 a[4], b[2];
+    u32x4 a[WNB], b[WMB];
   };
   int rd_slot = 0;   // LDS slot of the stage whose fragments are read next
   auto read_half = [&](int ks, Half& f) __attribute__((always_inline)) {
     const uint32_t so = (uint32_t)rd_slot * GM_STAGE;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) f.a[a] = lds_load<u32x4>(fa[a][ks] + so);
+    for (int a = 0; a < WNB; ++a) f.a[a] = lds_load<u32x4>(fa[a][ks] + so);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) f.b[b] = lds_load<u32x4>(fb[b][ks] + so);
+    for (int b = 0; b < WMB; ++b) f.b[b] = lds_load<u32x4>(fb[b][ks] + so);
   };
   auto mfmas = [&](const Half& f) __attribute__((always_inline)) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < WNB; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < WMB; ++b)
         acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, f.a[a]),
                                                             __builtin_bit_cast(bf16x8, f.b[b]), acc[a][b], 0, 0, 0);
   };
@@ -266,10 +268,10 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
   // beta * y (rounded once, after the addition).
   constexpr bool STG16 = OUT_BF16 && !ACC;
   constexpr int STG_COLS = STG16 ? 64 : 32;
-  // Rows row0 .. row0 + 31 of the staged block, STG_COLS columns from output
-  // column col0, to global memory: lane L stores chunk L % 8 of rows L / 8 +
+  // Rows row0 .. row0 + 31 of the staged block, `width` (at most STG_COLS)
+  // columns from output column col0, to global memory: lane L stores chunk L % 8 of rows L / 8 +
   // 8 j. Rows past m and chunks past n are dropped.
-  auto flush = [&](int64_t row0, int col0) __attribute__((always_inline)) {
+  auto flush = [&](int64_t row0, int col0, int width) __attribute__((always_inline)) {
     constexpr int EPC = STG16 ? 8 : 4;   // elements per 16-byte staged chunk
     const int c = lane & 7;
     const int col = col0 + c * EPC;
@@ -278,7 +280,7 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
       const int r = (lane >> 3) + 8 * j;
       const u32x4 v = lds_load<u32x4>(stg_at(r, c));
       const int64_t row = row0 + r;
-      if (row < p.m && col < p.n) {
+      if (row < p.m && col < p.n && c * EPC < width) {
         char* dst = p.y + (row * p.ys + col) * (OUT_BF16 ? 2 : 4);
         if constexpr (STG16) {
           *reinterpret_cast<u32x4*>(dst) = v;
@@ -315,8 +317,8 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
       lds_store<u32x4>(stg_at(l32, chunk_col >> 2), __builtin_bit_cast(u32x4, v));
     }
   };
-  // tile done: acc[a][b][4 * g + e] is product (row wm*64 + b*32 + l32,
-  // w row wn*128 + a*32 + 8*g + 4*hf + e) of the tile
+  // tile done: acc[a][b][4 * g + e] is product (row (wm*WMB + b)*32 + l32,
+  // w row (wn*WNB + a)*32 + 8*g + 4*hf + e) of the tile
   auto tile_end = [&]() __attribute__((always_inline)) {
     if (++mm_ks != kst) return;
     mm_ks = 0;
@@ -324,15 +326,15 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
     int nt;
     tile_of(mm_j++, &mt, &nt);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int64_t row0 = mt * GM_BM + wm * 64 + b * 32;
+    for (int b = 0; b < WMB; ++b) {
+      const int64_t row0 = mt * GM_BM + (wm * WMB + b) * 32;
       if constexpr (EPI == EPI_GEGLU) {
-        // block wn*4 + a: gate rows 0-15 and their up rows 16-31 give output
-        // columns 16 (wn*4 + a) + 0..15 of the tile: all four blocks are 64
-        // bf16 or f32 columns, staged 128 bytes (32 f32 columns) at a time
-        constexpr int PER = STG_COLS / 16;   // a-blocks (16 outputs each) per staging
+        // block wn*WNB + a: gate rows 0-15 and their up rows 16-31 give output
+        // columns 16 (wn*WNB + a) + 0..15 of the tile, staged up to 128 bytes
+        // (64 bf16 or 32 f32 columns) at a time
+        constexpr int PER = STG_COLS / 16 < WNB ? STG_COLS / 16 : WNB;   // a-blocks (16 outputs each) per staging
 #pragma unroll
-        for (int a0 = 0; a0 < 4; a0 += PER) {
+        for (int a0 = 0; a0 < WNB; a0 += PER) {
 #pragma unroll
           for (int a = a0; a < a0 + PER; ++a)
 #pragma unroll
@@ -343,12 +345,12 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
                 v[e] = gelu_tanh(p.alpha * acc[a][b][4 * g + e]) * (p.alpha * acc[a][b][4 * (g + 2) + e]);
               put4((a - a0) * 16 + 8 * g + 4 * hf, v);
             }
-          flush(row0, nt * BNO + wn * 64 + a0 * 16);
+          flush(row0, nt * BNO + (wn * WNB + a0) * 16, PER * 16);
         }
       } else {
-        constexpr int PER = STG_COLS / 32;   // a-blocks (32 columns each) per staging
+        constexpr int PER = STG_COLS / 32 < WNB ? STG_COLS / 32 : WNB;   // a-blocks (32 columns each) per staging
 #pragma unroll
-        for (int a0 = 0; a0 < 4; a0 += PER) {
+        for (int a0 = 0; a0 < WNB; a0 += PER) {
 #pragma unroll
           for (int a = a0; a < a0 + PER; ++a)
 #pragma unroll
@@ -356,7 +358,7 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
               f32x4 v;
               if constexpr (EPI == EPI_GELU_MUL) {
                 const int64_t row = row0 + l32;
-                const int col = nt * BNO + wn * 128 + a * 32 + 8 * g + 4 * hf;
+                const int col = nt * BNO + (wn * WNB + a) * 32 + 8 * g + 4 * hf;
                 bf16x4 mv = {};
                 if (row < p.m && col < p.n) mv = *reinterpret_cast<const bf16x4*>(p.mul + (row * p.ms + col) * 2);
 #pragma unroll
@@ -367,14 +369,14 @@ __global__ __launch_bounds__(GemmShapeOf<SH>::NW * 64, GemmShapeOf<SH>::WPC) voi
               }
               put4((a - a0) * 32 + 8 * g + 4 * hf, v);
             }
-          flush(row0, nt * BNO + wn * 128 + a0 * 32);
+          flush(row0, nt * BNO + (wn * WNB + a0) * 32, PER * 32);
         }
       }
     }
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < WNB; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = zero;
+      for (int b = 0; b < WMB; ++b) acc[a][b] = zero;
   };
   // One iteration per stage s, with h0 holding its first k step's operands:
   // read its second k step's operands while the first step's MFMAs run;
@@ -412,6 +414,8 @@ const void* gemm_fn() {
 template <int SH>
 int gemm_launch_shape(GemmParams p, int epi, bool bf, bool acc, int64_t m, int64_t k, int cus, void* stream) {
   using C = GemmShapeOf<SH>;
+  const int bno = epi == EPI_GEGLU ? C::BN / 2 : C::BN;
+  p.n_tiles_n = (p.n + bno - 1) / bno;
   p.n_tiles = ((m + C::BM - 1) / C::BM) * p.n_tiles_n;
   p.per_xcd = (p.n_tiles + GM_XCDS - 1) / GM_XCDS;
   // C::WPC workgroups per CU, at most one per tile of an XCD's range
@@ -443,6 +447,42 @@ int gemm_launch_shape(GemmParams p, int epi, bool bf, bool acc, int64_t m, int64
   return INL_OK;
 }
 
+// The shape with the least estimated time: q tiles one after another on the
+// fullest CU, each kst stages of `stage` us and `drain` us of epilogue (halved
+// for bf16 outputs: it is the time of the stores). Fitted to the seven
+// EmbeddingGemma projections at 1 to 60,000 rows (k 256 to 1,152, n 256 to
+// 2,304): us per GEMM of the shapes 0 / 1 / 2 / 3
+//   768 -> 768 f32:   1 row 18.1 / 13.7 / 9.8 / 6.9,   2,500 20.1 / 15.7 / 11.4 / 10.3,
+//                     10,000 23.4 / 22.5 / 22.7 / 28.4, 60,000 91 / 101 / 115 / 184
+//   GEGLU 768 -> 1,152: 1,000 rows 20.0 / 15.2 / 11.3 / 14.1, 5,000 25.1 / 27.0 / 28.8 / 42.1
+//   256 -> 768 f32:   21,658 rows 28.9 / 22.3 / 20.5 / 27.0
+// Before, all outputs wider than 256 ran on shape 0 and the others on shape 1.
+int pick_shape(int epi, int64_t m, int64_t n, int64_t k, bool bf, int cus) {
+  struct Cost {
+    int bn, bm, wpc;
+    float stage, drain, alone;   // alone: us per stage of a tile that has its CU to itself
+  };
+  static const Cost costs[4] = {{GemmShapeOf<0>::BN, GemmShapeOf<0>::BM, 1, 0.55f, 13.f, 0.55f},
+                                {GemmShapeOf<1>::BN, GemmShapeOf<1>::BM, 2, 0.58f, 4.5f, 0.58f},
+                                {GemmShapeOf<2>::BN, GemmShapeOf<2>::BM, 2, 0.28f, 2.4f, 0.28f},
+                                {GemmShapeOf<3>::BN, GemmShapeOf<3>::BM, 2, 0.106f, 0.6f, 0.157f}};
+  const float kst = (float)(k / GM_BK);
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < 4; ++i) {
+    const Cost& c = costs[i];
+    const int64_t bno = epi == EPI_GEGLU ? c.bn / 2 : c.bn;
+    const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + bno - 1) / bno);
+    const float q = (float)((tiles + cus - 1) / cus), rounds = (float)((tiles + (int64_t)cus * c.wpc - 1) / ((int64_t)cus * c.wpc));
+    const float t = std::max(rounds * kst * c.alone, q * (kst * c.stage + (bf ? 0.53f : 1.f) * c.drain));
+    if (i == 0 || t < least) {
+      least = t;
+      best = i;
+    }
+  }
+  return best;
+}
+
 // Launch for every epilogue; `n` is the output width (GEGLU: w has 2n rows).
 int gemm_launch(int epi, int64_t m, int64_t n, int64_t k, const void* x, int64_t x_stride, const void* w,
                 int64_t w_stride, const void* mul, int64_t mul_stride, int32_t out_dtype, void* y, int64_t y_stride,
@@ -463,12 +503,11 @@ int gemm_launch(int epi, int64_t m, int64_t n, int64_t k, const void* x, int64_t
   if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 15) || ((uintptr_t)mul & 7))
     return fail(INL_E_INVALID, "gemm: x, w and y must be 16-byte aligned, the multiplier 8-byte aligned");
   // each tile's descriptor spans at most 256 rows of x or w
-  if ((int64_t)256 * xs * 2 >= ((int64_t)1 << 32) || (int64_t)GM_BN * ws * 2 >= ((int64_t)1 << 32))
+  if ((int64_t)256 * xs * 2 >= ((int64_t)1 << 32) || (int64_t)256 * ws * 2 >= ((int64_t)1 << 32))
     return fail(INL_E_UNSUPPORTED, "gemm: row strides too large for a tile's 32-bit buffer range");
   int dev = 0, cus = 0;
   INL_HIP_TRY(hipGetDevice(&dev));
   INL_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int bno = epi == EPI_GEGLU ? GM_BN / 2 : GM_BN;
   GemmParams p{};
   p.x = (const char*)x;
   p.w = (const char*)w;
@@ -483,10 +522,14 @@ int gemm_launch(int epi, int64_t m, int64_t n, int64_t k, const void* x, int64_t
   p.ys = ys;
   p.alpha = alpha;
   p.beta = beta;
-  p.n_tiles_n = (int32_t)((n + bno - 1) / bno);
   const bool bf = out_dtype == INL_BF16, acc = beta != 0.f;
-  if (p.n_tiles_n == 1) return gemm_launch_shape<1>(p, epi, bf, acc, m, k, cus, stream);
-  return gemm_launch_shape<0>(p, epi, bf, acc, m, k, cus, stream);
+  const int sh = pick_shape(epi, m, n, k, bf, cus);
+  switch (sh) {
+    case 0: return gemm_launch_shape<0>(p, epi, bf, acc, m, k, cus, stream);
+    case 1: return gemm_launch_shape<1>(p, epi, bf, acc, m, k, cus, stream);
+    case 2: return gemm_launch_shape<2>(p, epi, bf, acc, m, k, cus, stream);
+    default: return gemm_launch_shape<3>(p, epi, bf, acc, m, k, cus, stream);
+  }
 }
 
 }  // namespace

@@ -189,3 +189,43 @@ def test_gated_gemm_config3_full_size(mode, cuda, inl):
     got = y[ri, :n].double().cpu().numpy()
     tol = 2.0 ** -8 * np.abs(ref) + 1e-5 * np.abs(ref).max()
     assert (np.abs(got - ref) <= tol).all(), np.abs(got - ref).max()
+
+
+# Every kernel shape and epilogue: row counts that the cost rule sends to the
+# 64 x 64, 128 x 128, 256 x 128 and 256 x 256 tiles, each with ragged last
+# tiles in m and n. Against f64 products of the same bf16 values, the bound of
+# the tests above (bf16 rounding of the output, 1e-5 of the largest |y|).
+SHAPE_CASES = [(1, 40, 32), (63, 72, 96), (65, 136, 768), (1000, 1160, 768), (2500, 1160, 768), (5000, 776, 768),
+               (5000, 1288, 768), (9999, 776, 256), (9000, 1288, 768), (20001, 264, 256)]
+
+
+@pytest.mark.parametrize("epi", ["plain", "geglu", "gelu_mul"])
+@pytest.mark.parametrize("m,n,k", SHAPE_CASES)
+def test_every_kernel_shape(m, n, k, epi, cuda, inl):
+    import torch
+    gen = torch.Generator(device=cuda).manual_seed(m + n)
+    rows = 2 * n if epi == "geglu" else n
+    x = torch.randn(m, k, generator=gen, device=cuda).to(torch.bfloat16)
+    w = (torch.randn(rows, k, generator=gen, device=cuda) * k ** -0.5).to(torch.bfloat16)
+    mul = torch.randn(m, n, generator=gen, device=cuda).to(torch.bfloat16)
+    print(f"case=gemm_shape {m}x{n}x{k} {epi}", flush=True)
+    gelu = lambda t: torch.nn.functional.gelu(t, approximate="tanh")
+    p = x.double() @ w.double().T
+    if epi == "plain":
+        ref = p
+    elif epi == "geglu":
+        ref = gelu(p[:, :n]) * p[:, n:]
+    else:
+        ref = gelu(p) * mul.double()
+    for od in (torch.float32, torch.bfloat16):
+        out = torch.full((m + 1, n), float("nan"), dtype=od, device=cuda)
+        y = out[:m]
+        if epi == "plain":
+            inl.gemm_bf16(x, w, out=y)
+        else:
+            inl.gemm_bf16_gated(x, w, epi, mul=mul if epi == "gelu_mul" else None, out=y)
+        torch.cuda.synchronize()
+        assert torch.isnan(out[m].float()).all(), "a row past m was written"
+        err = (y.double() - ref).abs()
+        bound = 1e-5 * ref.abs().max() + (ref.abs() * 2 ** -8 if od == torch.bfloat16 else 0)
+        assert (err <= bound).all(), f"{od}: max error {err.max().item():.3g}"
