@@ -17,6 +17,11 @@
 //     residual += m . Wdown^T                               (beta 1)
 //   embeddings = l2(rms_norm(residual[last row]) * norm)    (inl_pool_last_fwd)
 //
+// That is the general sequence. Batches of a few rows run on five launches a
+// layer of their own (skinny.hip), and f32 batches from a few hundred rows up
+// on the library's f32 GEMM, with SwiGLU in its epilogue and the residual
+// addition in the row norm that follows (gemm_f32.hip).
+//
 // The attention schedule is planned once per call into the workspace and
 // reused by every layer; nothing is allocated per call.
 //
@@ -42,6 +47,7 @@
 
 #include "../../include/inl_encoder.h"
 #include "inl_common.hpp"
+#include "gemm_f32.hpp"
 #include "skinny.hpp"
 
 struct inl_qwen3 {
@@ -68,6 +74,13 @@ struct inl_qwen3 {
 namespace inl {
 
 namespace {
+
+// f32 batches of more rows than this run on the library's own GEMM, smaller
+// ones on hipBLASLt (us per encode of the 0.6B shape, own / hipBLASLt: 400 rows
+// 5,109 / 4,993, 512 rows 5,357 / 6,405, 800 6,986 / 7,811, 1,024 7,505 /
+// 11,350, 2,048 12,408 / 15,582: a 128-row tile's k loop is serial, and few
+// tiles leave CUs idle).
+constexpr int64_t OWN_GEMM_ROWS = 464;
 
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
@@ -352,6 +365,10 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
   rc = inl_linear_workspace_size(&gws_bytes);
   if (rc) return rc;
 
+  int dev = 0, cus = 0;
+  INL_HIP_TRY(hipGetDevice(&dev));
+  INL_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+
   // the attention plan of this batch, used by every layer
   const int dt = c.dtype, es = dtype_size(dt);
   const int64_t qd = (int64_t)c.heads * c.head_dim, kvd = (int64_t)c.kv_heads * c.head_dim;
@@ -401,6 +418,12 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
     return rc;
   }
 
+  // (a projection's parts go to the workspace that hipBLASLt would get)
+  const bool own = !few && dt == INL_F32 && gemm_f32_fits(c.hidden, (int32_t)qkv_w, (int32_t)qd, c.intermediate) &&
+                   (size_t)n * c.hidden * 4 <= gws_bytes && n > OWN_GEMM_ROWS;
+  const int o_parts = own ? gemm_f32_splits(n, c.hidden, (int32_t)qd, cus, gws_bytes) : 1;
+  const int d_parts = own ? gemm_f32_splits(n, c.hidden, c.intermediate, cus, gws_bytes) : 1;
+
   // the launch sequence, onto stream `sq` (the caller's, or the capture stream)
   auto sequence = [&](void* sq) -> int {
   inl_norm_rope_desc nr{};
@@ -440,8 +463,11 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
                                   resid, c.hidden, hf, to_qkv, sq);
       continue;
     }
-    rc = inl_rms_norm_rows_fwd(n, c.hidden, resid, c.hidden, w.input_norm, dt, c.eps, dt, x, c.hidden, stream);
-    if (!rc) rc = inl_linear_fwd(n, qkv_w, c.hidden, dt, x, c.hidden, w.qkv_proj, c.hidden, dt, A, L.a_w, 1.f, 0.f,
+    if (!own || i == 0)
+      rc = inl_rms_norm_rows_fwd(n, c.hidden, resid, c.hidden, w.input_norm, dt, c.eps, dt, x, c.hidden, stream);
+    if (!rc && own) rc = gemm_f32_launch(n, (int32_t)qkv_w, c.hidden, (const float*)x, c.hidden, (const float*)w.qkv_proj,
+                                         GF_STORE, 1, (float*)A, L.a_w, (hipStream_t)stream);
+    else if (!rc) rc = inl_linear_fwd(n, qkv_w, c.hidden, dt, x, c.hidden, w.qkv_proj, c.hidden, dt, A, L.a_w, 1.f, 0.f,
                                  gws, gws_bytes, stream);
     if (!rc && c.heads % 4 == 0) {
       // q and k heads are adjacent in the QKV row: one launch, k_norm from head `heads` on
@@ -458,6 +484,21 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
       }
     }
     if (!rc) rc = inl_attn_fwd(plan, A, A + qd * es, A + (qd + kvd) * es, B, stream);
+    if (own) {
+      hipStream_t sq = (hipStream_t)stream;
+      float* part = (float*)gws;
+      const float* next = i + 1 < c.layers ? (const float*)e->layers[i + 1].input_norm : nullptr;
+      if (!rc) rc = gemm_f32_launch(n, c.hidden, (int32_t)qd, (const float*)B, L.b_w, (const float*)w.o_proj, GF_PART,
+                                    o_parts, part, c.hidden, sq);
+      if (!rc) rc = add_norm_launch(n, c.hidden, resid, part, o_parts, (const float*)w.post_attention_norm, c.eps,
+                                    (float*)x, sq);
+      if (!rc) rc = gemm_f32_launch(n, c.intermediate, c.hidden, (const float*)x, c.hidden,
+                                    (const float*)w.gate_up_proj, GF_SWIGLU, 1, (float*)B, L.b_w, sq);
+      if (!rc) rc = gemm_f32_launch(n, c.hidden, c.intermediate, (const float*)B, L.b_w, (const float*)w.down_proj,
+                                    GF_PART, d_parts, part, c.hidden, sq);
+      if (!rc) rc = add_norm_launch(n, c.hidden, resid, part, d_parts, next, c.eps, (float*)x, sq);
+      continue;
+    }
     if (!rc) rc = inl_linear_fwd(n, c.hidden, qd, dt, B, L.b_w, w.o_proj, qd, INL_F32, resid, c.hidden, 1.f, 1.f,
                                  gws, gws_bytes, stream);
     if (!rc) rc = inl_rms_norm_rows_fwd(n, c.hidden, resid, c.hidden, w.post_attention_norm, dt, c.eps, dt, x,

@@ -49,3 +49,25 @@ def test_few_rows_against_oracle(shape, lengths, dtype, cuda, inl):
         else:
             assert cos.min() >= 0.999
     enc.close()
+
+
+# f32 batches above 464 rows run on the library's own f32 GEMM: row counts at
+# the edges of its 128-row tiles and of the path, and widths with other part
+# counts. The tolerance of the general path.
+@pytest.mark.parametrize("shape,lengths", [("0.6B", [465]), ("0.6B", [200, 312]), ("0.6B", [300, 200, 140, 1]),
+                                           ("group1", [500, 13]), ("group4", [512, 257])])
+def test_f32_gemm_rows_against_oracle(shape, lengths, cuda, inl):
+    import torch
+    cfg = oq.Qwen3Config(vocab=512, layers=2, **SHAPES[shape])
+    w = oq.random_weights(cfg, seed=12)
+    wd = {k: torch.from_numpy(np.ascontiguousarray(v)).to(cuda) for k, v in w.items()}
+    rng = np.random.default_rng(sum(lengths))
+    cu = oa.cu_from_lengths(lengths)
+    ids = rng.integers(0, cfg.vocab, sum(lengths))
+    print(f"case=f32_gemm {shape} {lengths}", flush=True)
+    enc = inl.Qwen3Encoder(cfg, wd, max_positions=512)
+    got = enc.encode(ids, cu.tolist()).cpu().numpy().astype(np.float64)
+    enc.close()
+    ref = oq.encode(w, cfg, ids, cu)
+    cos = (got * ref).sum(1) / np.linalg.norm(got, axis=1) / np.linalg.norm(ref, axis=1)
+    assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4
