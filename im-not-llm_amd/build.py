@@ -51,7 +51,8 @@ EXTRA = {
 # spill could store that register, or hand it to another value, while the
 # load is still in flight. Their kernels must use no scratch; the build reads
 # the compiler's resource-usage remarks and fails if any of them does.
-NO_SCRATCH = {"attn_pp.hip", "attn_pp64.hip", "attn_wide.hip", "gemm.hip", "splade_decoder.hip"}
+NO_SCRATCH = {"attn_pp.hip", "attn_pp64.hip", "attn_wide.hip", "gdn_chunk.hip", "gemm.hip", "gemm_f32.hip",
+              "splade_decoder.hip"}
 RESOURCE_REMARKS = ["-Rpass-analysis=kernel-resource-usage", "-fno-caret-diagnostics"]
 # The same sources are also compiled to a device assembly listing, which
 # asmcheck.py walks for instructions that name a register an inline-asm
