@@ -35,7 +35,16 @@
 // 8x the P precision of bf16: a causal row that sees two keys of comparable
 // weight would otherwise carry up to ~4e-3 of P rounding error. The flag
 // INL_ATTN_PV_BF16 keeps V and P in bf16 instead (any V range, coarser P).
-// f32 inputs use v_mfma_f32_32x32x2_f32 throughout.
+// f32 inputs take the same bf16 instruction: Q, K, V and P are each the sum of
+// three bf16 values (8 + 8 + 8 significand bits, rounded to nearest), and the
+// six of the nine products above 2^-26 of the whole are summed in f32, the
+// leading ones and the small ones apart. They are exact, so a product carries
+// f32's precision, at six times the bf16 instruction's cost and 0.75 of the
+// f32 one's, with an eighth of its accumulator roundings. K and V are split
+// once per workgroup, while they are staged; the planes of one tile fill LDS
+// (96 KiB at head_dim 128), so the next tile waits in registers. Against
+// v_mfma_f32_32x32x2_f32: 32 passages, 8,110 tokens, 16 / 8 heads of 128
+// causal 312 -> 222 us, error against f64 3.0e-7 -> 1.3e-7.
 
 #include <algorithm>
 #include <cmath>
@@ -73,8 +82,51 @@ __device__ __forceinline__ int vcol(int key4) {
   }
 }
 
+// Four f32 values as three bf16 parts each (8 bytes a part).
+__device__ __forceinline__ void split4(const f32x4& x, u32x2 (&o)[3]) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    f32x2 r = {x[2 * j], x[2 * j + 1]};
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+      o[n][j] = u;
+      if (n < 2) {
+        r[0] -= __builtin_bit_cast(float, u << 16);
+        r[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+      }
+    }
+  }
+}
+// The MFMA operand of eight, in three parts.
+__device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, bf16x8 (&o)[3]) {
+  u32x2 x[3], y[3];
+  split4(a, x);
+  split4(b, y);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) o[n] = __builtin_bit_cast(bf16x8, (u32x4){x[n][0], x[n][1], y[n][0], y[n][1]});
+}
+// hi + lo += a . b of operands in three parts.
+__device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x16& hi, f32x16& lo) {
+#pragma unroll
+  for (int d = 2; d > 0; --d)
+#pragma unroll
+    for (int i = 0; i <= d; ++i) lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[d - i], lo, 0, 0, 0);
+  hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], hi, 0, 0, 0);
+}
+// LDS address, inside the planes of a tile, of part 0 of fragment `frag` (32
+// rows x 16 terms in operand order, 1 KiB a part, the three parts in a row):
+// the 16 bytes of (row, half). `x` swizzles the rows so that a wave's writes,
+// 8 bytes a lane, spread over the banks.
+__device__ __forceinline__ int frag_at(int frag, int row, int hf, int x) {
+  return frag * 3072 + (hf * 32 + (row ^ x)) * 16;
+}
+
+// (head_dim 64: two waves per SIMD, 256 registers each. In f32 the split
+// otherwise takes 337, and the short units of a local band then run one
+// workgroup per CU: 106 against 74 us on 16 texts of up to 1,000.)
 template <typename E, int D, int BN, int NW, bool PV16>
-__global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
+__global__ __launch_bounds__(NW * 64, D <= 64 ? 2 : 1) void attn_fwd_kernel(AttnParams p) {
   typedef typename PvType<E, PV16>::T PT;
   constexpr int NT = NW * 64;
   constexpr int ES = (int)sizeof(E);
@@ -89,6 +141,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
   constexpr int VPT = (NVU + NT - 1) / NT;
   constexpr int NKB = BN / 32;          // 32-key blocks per tile
   constexpr int NDB = D / 32;           // 32-wide d blocks of the output
+  constexpr int NKJ = D / 16;           // f32: 16-dim steps of QK^T
+  constexpr int PLANES = BN * D * 6;    // f32: three bf16 parts of K, or of V^T
   static_assert(CHK >= 8 && (VROW / 16) >= 8, "swizzle needs 8 chunks per row");
   static_assert(BN % 32 == 0 && D % 32 == 0, "tile shape");
 
@@ -136,6 +190,14 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
     qreg[i] = z;
   }
 
+  // f32: Q^T in parts. Term 4 h + e of step j in lane half hf is element e of
+  // the row's 16-byte chunk 4 j + 2 h + hf, for K as well.
+  bf16x8 qp[ES == 4 ? NKJ : 1][3];
+  if constexpr (ES == 4)
+#pragma unroll
+    for (int j = 0; j < NKJ; ++j)
+      split8(__builtin_bit_cast(f32x4, qreg[2 * j]), __builtin_bit_cast(f32x4, qreg[2 * j + 1]), qp[j]);
+
   f32x16 oacc[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i)
@@ -182,14 +244,23 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
   };
 
   auto store_tile = [&](int buf) {
-    char* sK = smem + buf * 2 * KT_BYTES;
-    char* sV = sK + KT_BYTES;
+    char* sK = smem + (ES == 4 ? 0 : buf * 2 * KT_BYTES);
+    char* sV = sK + (ES == 4 ? PLANES : KT_BYTES);
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int id = tid + i * NT;
       if (NKC % NT == 0 || id < NKC) {
         const int row = id / CHK, c = id % CHK;
-        *reinterpret_cast<u32x4*>(sK + swz(row, c, KROW)) = kst[i];
+        if constexpr (ES == 4) {
+          const int j = c >> 2, half = c & 1;
+          u32x2 o[3];
+          split4(__builtin_bit_cast(f32x4, kst[i]), o);
+          char* dst = sK + frag_at((row >> 5) * NKJ + j, row & 31, half, (2 * j + half) & 31) + ((c >> 1) & 1) * 8;
+#pragma unroll
+          for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(dst + n * 1024) = o[n];
+        } else {
+          *reinterpret_cast<u32x4*>(sK + swz(row, c, KROW)) = kst[i];
+        }
       }
     }
 #pragma unroll
@@ -223,12 +294,20 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
             *reinterpret_cast<u32x2*>(sV + swz(dd, col >> 3, VROW) + (col & 7) * 2) = val;
           }
         } else {
-          // 4 keys x 4 d (f32) -> for each d, 4 consecutive keys (16 bytes)
+          // 4 keys x 4 d (f32) -> for each d, 4 consecutive keys in parts.
+          // Term 4 h + e of step i of key block kb in lane half hf is key
+          // 32 kb + 16 i + 8 h + 4 hf + e: the order of the S^T accumulator.
+          const int kb = g >> 3, step = (g >> 2) & 1, h = (g >> 1) & 1, half = g & 1;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int dd = c * 4 + e;
-            u32x4 val = {vst[i][0][e], vst[i][1][e], vst[i][2][e], vst[i][3][e]};
-            *reinterpret_cast<u32x4*>(sV + swz(dd, col >> 2, VROW)) = val;
+            const int dd = c * 4 + e, db = dd >> 5;
+            u32x2 o[3];
+            const f32x4 keys = {__builtin_bit_cast(f32x4, vst[i][0])[e], __builtin_bit_cast(f32x4, vst[i][1])[e],
+                                __builtin_bit_cast(f32x4, vst[i][2])[e], __builtin_bit_cast(f32x4, vst[i][3])[e]};
+            split4(keys, o);
+            char* dst = sV + frag_at((db * NKB + kb) * 2 + step, dd & 31, half, db & 3) + h * 8;
+#pragma unroll
+            for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(dst + n * 1024) = o[n];
           }
         }
       }
@@ -250,8 +329,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
 
     const int kt0 = t * BN;
     if (active && kt0 < khi && kt0 + BN > klo) {
-      const char* sK = smem + buf * 2 * KT_BYTES;
-      const char* sV = sK + KT_BYTES;
+      const char* sK = smem + (ES == 4 ? 0 : buf * 2 * KT_BYTES);
+      const char* sV = sK + (ES == 4 ? PLANES : KT_BYTES);
 
       // ---- S^T = K . Q^T ----
       f32x16 sacc[NKB];
@@ -270,16 +349,21 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
             }
           }
         } else {
+          f32x16 lo;
 #pragma unroll
-          for (int g = 0; g < D / 8; ++g) {
-            if (g * 8 < hd) {
-              f32x4 a = *reinterpret_cast<const f32x4*>(sK + swz(krow, 2 * g + hf, KROW));
-              f32x4 b = __builtin_bit_cast(f32x4, qreg[g]);
+          for (int r = 0; r < 16; ++r) lo[r] = 0.f;
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], sacc[kb], 0, 0, 0);
+          for (int j = 0; j < NKJ; ++j) {
+            if (j * 16 < hd) {
+              const char* src0 = sK + frag_at(kb * NKJ + j, lq, hf, (2 * j + hf) & 31);
+              bf16x8 a[3];
+#pragma unroll
+              for (int n = 0; n < 3; ++n) a[n] = *reinterpret_cast<const bf16x8*>(src0 + n * 1024);
+              mfma_split(a, qp[j], sacc[kb], lo);
             }
           }
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sacc[kb][r] += lo[r];
         }
       }
 
@@ -362,25 +446,39 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(AttnParams p) {
         for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) l_i += sacc[kb][r];
+        bf16x8 pk[NKB * 2][3];
+#pragma unroll
+        for (int ks = 0; ks < NKB * 2; ++ks) {
+          f32x4 a, b;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            a[e] = sacc[ks >> 1][8 * (ks & 1) + e];
+            b[e] = sacc[ks >> 1][8 * (ks & 1) + 4 + e];
+          }
+          split8(a, b, pk[ks]);
+        }
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
           if (db * 32 < hd) {
-            const int vrow = db * 32 + lq;
+            f32x16 lo;
 #pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
+            for (int r = 0; r < 16; ++r) lo[r] = 0.f;
 #pragma unroll
-              for (int q4 = 0; q4 < 4; ++q4) {
-                f32x4 a = *reinterpret_cast<const f32x4*>(sV + swz(vrow, 8 * kb + 4 * hf + q4, VROW));
+            for (int ks = 0; ks < NKB * 2; ++ks) {
+              const char* src0 = sV + frag_at(db * NKB * 2 + ks, lq, hf, db & 3);
+              bf16x8 a[3];
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], sacc[kb][4 * q4 + e], oacc[db], 0, 0, 0);
-              }
+              for (int n = 0; n < 3; ++n) a[n] = *reinterpret_cast<const bf16x8*>(src0 + n * 1024);
+              mfma_split(a, pk[ks], oacc[db], lo);
             }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[db][r] += lo[r];
           }
         }
       }
     }
 
+    if constexpr (ES == 4) __syncthreads();   // every wave has read the one tile LDS holds
     if (more) store_tile(buf ^ 1);
     __syncthreads();
   }
@@ -588,7 +686,8 @@ int unit_weight(const KernelCfg& cfg, const inl_attn_desc* d, int T, int q0, int
 
 template <typename E, int D, int BN, int NW, bool PV16>
 KernelCfg make_cfg(const char* name) {
-  return KernelCfg{attn_fwd_kernel<E, D, BN, NW, PV16>, D, BN, NW, 4 * BN * D * (int)sizeof(E), 32, false, false,
+  return KernelCfg{attn_fwd_kernel<E, D, BN, NW, PV16>, D, BN, NW,
+                   sizeof(E) == 4 ? 12 * BN * D : 4 * BN * D * (int)sizeof(E), 32, false, false,
                    name};
 }
 
@@ -1037,7 +1136,7 @@ void assign_units(const std::vector<CostedItem>& items, int n_hg, int gpk, Sched
 // Key-range split for the generic f32 kernel. Its workgroups hold one query
 // block each and walk the block's key tiles in order, so a small batch
 // (fewer workgroups than the GPU holds at once) takes as long as its longest
-// block: 4 tiles of about 7 us each for a 256-token causal text at head_dim
+// block: 4 tiles of about 5 us each for a 256-token causal text at head_dim
 // 128. Cutting blocks into parts of at most `c` tiles, each part a workgroup
 // of its own, and merging the parts afterwards shortens that. `c` minimises
 // an estimate in tile times: the workgroups, longest first, dispatched to

@@ -252,3 +252,29 @@ def test_pv_fp16_range_contract(cuda, inl):
     print(f"pv_bf16: worst error / bound = {ratio:.3f}", flush=True)
     assert ratio <= 1.0
     assert np.abs(got[t1]).max() > 1000.0  # the large key is really in play
+
+
+@pytest.mark.parametrize("d", [8, 24, 40, 64, 72, 96, 128, 136, 200, 256])
+@pytest.mark.parametrize("causal,window", [(True, -1), (False, 33)])
+def test_f32_parts_every_head_dim(d, causal, window, cuda, inl):
+    """f32 attention multiplies three bf16 parts of each value: head dims that
+    fill its 16-dim steps and compiled widths (64, 128, 256) and ones that do
+    not, text lengths around its 32- and 64-key tiles, values over ten orders of
+    magnitude. The oracle's f64 on the same f32 inputs; a product of parts is
+    off by at most 2^-24 of its factors, a sum of n of them by some sqrt(n)
+    2^-24: 2e-6 of the largest value of a text's head."""
+    import torch
+    lengths = [1, 31, 32, 65, 130]
+    hq, hkv = 4, 2
+    (q, k, v), (hq_, hk_, hv_) = _inputs(lengths, hq, hkv, d, d, torch.float32, torch, cuda, d ** -0.5)
+    scale_v = torch.logspace(-5, 5, sum(lengths), device=cuda)[:, None, None]
+    v = (v * scale_v).contiguous()
+    cu = oa.cu_from_lengths(lengths)
+    print(f"case=f32_parts d={d} causal={causal} window={window}", flush=True)
+    out = inl.varlen_attention(q, k, v, cu.tolist(), causal=causal, window=window).cpu().numpy()
+    ref = oa.varlen_attention(hq_, hk_, v.cpu().numpy().astype(np.float64), cu, causal=causal, window=window,
+                              scale=d ** -0.5)
+    for b in range(len(lengths)):
+        r = ref[cu[b]:cu[b + 1]]
+        bound = 2e-6 * np.abs(v[cu[b]:cu[b + 1]].cpu().numpy()).max()
+        assert np.abs(out[cu[b]:cu[b + 1]] - r).max() <= bound
