@@ -13,7 +13,7 @@
 //   S   <- e^(c_C) S + K^T (e^(c_C - c) U)
 //
 // Measured against the per-token kernel, rule alone, 16 heads, bf16: 16 texts
-// of 80 to 1,453 tokens 861 -> 264 us, 16 texts of 2,048 1,216 -> 510 us.
+// of 80 to 1,453 tokens 861 -> 243 us, 16 texts of 2,048 1,216 -> 462 us.
 //
 // Non-finite values: 0 times inf is NaN in a product, so an inf or NaN in a
 // token's row may reach earlier tokens of its own chunk and head as well.
@@ -348,7 +348,15 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnChunkParams p) {
   }
 }
 
-// LDS of gdn_chunk_rule: fragments of 1 KiB (16 bytes per lane).
+// LDS of gdn_chunk_rule: fragments of 1 KiB, 16 bytes per lane. Row i of lane
+// group g sits at slot 16 g + (i ^ x); x, a constant of the fragment and lane
+// group, spreads what a wave writes at a time over the banks: it loads whole
+// rows (a load of 16 bytes per lane from 16 rows runs at a quarter of the rate
+// of one from 4), so its lanes write one or two rows of many fragments. Against
+// loads in operand order: gdn_chunk_rule 219 -> 197 us at 16 texts of 80 to
+// 1,453 tokens, 16 heads, bf16. f32 loads K and Q in operand order still: their
+// three parts a value leave no registers for a second layout.
+__device__ __forceinline__ int gc_slot(int g, int i, int x) { return (16 * g + (i ^ x)) * 16; }
 template <typename T>
 struct GcLds {
   static constexpr int C = gc_len<T>(), RB = C / 16, TS = C / 32, NP = gc_parts<T>();
@@ -365,9 +373,8 @@ template <typename T>
 __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p) {
   using L = GcLds<T>;
   constexpr int C = L::C, RB = L::RB, TS = L::TS, NP = L::NP;
-  constexpr int FK = RB * 4 / GC_WAVES;   // K (and Q) fragments a wave stages
+  constexpr int FK = RB * 4 / GC_WAVES;   // KiB of K (and Q) a wave stages
   constexpr int FT = 8 * TS / GC_WAVES;   // K^T fragments
-  constexpr int FP = RB * TS;             // T (and P) fragments in all: wave w stages fragment w
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int h = blockIdx.x, b = blockIdx.y;
   int64_t begin, end;
@@ -381,13 +388,21 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
   const uint32_t q_off = (uint32_t)kh * GC_D, k_off = (uint32_t)(p.nk + kh) * GC_D;
   const uint32_t v_off = (uint32_t)2 * p.nk * GC_D + (uint32_t)h * GC_D + 16 * wave + i16;
   const uint32_t ms = (uint32_t)p.ms, os = (uint32_t)p.os;
-  auto frag = [&](int base, int i) __attribute__((always_inline)) {
-    return reinterpret_cast<bf16x8*>(smem + base + i * 1024 + lane * 16);
+  // fragment i of an array, this lane's 16 bytes
+  auto frag = [&](int base, int i, int x) __attribute__((always_inline)) {
+    return reinterpret_cast<bf16x8*>(smem + base + i * 1024 + gc_slot(g, i16, x));
   };
+  // the swizzles: K and Q of step s, K^T of block db, T and P of step ts
+  auto x_k = [](int s) __attribute__((always_inline)) { return 4 * s; };
+  auto x_t = [](int db) __attribute__((always_inline)) { return 2 * db; };
+  auto x_l = [](int grp, int ts) __attribute__((always_inline)) { return 2 * grp | 8 * ts; };
 
   // registers of the chunk to come
+  // bf16: 2 x 4 whole rows of K and Q; f32: operands. T and P: RT x 2 rows.
+  constexpr int RT = C / 2 / GC_WAVES;
   Raw<T> rk[FK], rq[FK], rt[FT];
-  float rT[8], rP[8], rs[4];
+  f32x4 rl[RT];
+  float rs[4];
   T rv[RB][4];
   auto load_t = [&](__amdgpu_buffer_rsrc_t r, uint32_t off) __attribute__((always_inline)) {
     if constexpr (sizeof(T) == 2)
@@ -398,31 +413,34 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
     const int rows = (int)min((int64_t)C, end - t0);
     const __amdgpu_buffer_rsrc_t mr = gc_rows_of(p.mixed, t0, p.ms, rows, width, ES);
     const __amdgpu_buffer_rsrc_t orr = gc_rows_of(p.out, t0, p.os, rows, (int64_t)p.nv * GC_D, 4);
+    if constexpr (NP == 1) {
 #pragma unroll
-    for (int f = 0; f < FK; ++f) {
-      const int id = wave * FK + f, rb = id >> 2, s = id & 3;
-      const uint32_t at = (16 * rb + i16) * ms + 32 * s + 4 * g;
-      gc_load<T>(rk[f], mr, (at + k_off) * ES);
-      gc_load<T>(rq[f], mr, (at + q_off) * ES);
-    }
+      for (int f = 0; f < FK; ++f) {   // row 8 wave + 4 f + lane / 16, dims 8 (lane % 16) ..
+        const uint32_t at = (8 * wave + 4 * f + g) * ms + 8 * i16;
+        rk[f].v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(mr, (at + k_off) * ES, 0, 0));
+        rq[f].v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(mr, (at + q_off) * ES, 0, 0));
+      }
+    } else {
 #pragma unroll
-    for (int f = 0; f < FT; ++f) {
-      const int id = wave * FT + f, db = id / TS, ts = id % TS;
+      for (int f = 0; f < FK; ++f) {
+        const int id = wave * FK + f, rb = id >> 2, s = id & 3;
+        const uint32_t at = (16 * rb + i16) * ms + 32 * s + 4 * g;
+        gc_load<T>(rk[f], mr, (at + k_off) * ES);
+        gc_load<T>(rq[f], mr, (at + q_off) * ES);
+      }
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        rt[f].v[e] = load_t(mr, ((32 * ts + 16 * (e >> 2) + 4 * g + (e & 3)) * ms + k_off + 16 * db + i16) * ES);
-    }
-    {
-      const int id = wave < FP ? wave : 0, rb = id / TS, ts = id % TS;
-      const uint32_t at = ((16 * rb + i16) * os + (uint32_t)h * GC_D + 32 * ts + 4 * g) * 4;
+      for (int f = 0; f < FT; ++f) {
+        const int id = wave * FT + f, db = id / TS, ts = id % TS;
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(orr, at + 64 * hh, 0, 0));
-        const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(orr, at + 256 + 64 * hh, 0, 0));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { rT[4 * hh + e] = a[e]; rP[4 * hh + e] = q[e]; }
+        for (int e = 0; e < 8; ++e)
+          rt[f].v[e] = load_t(mr, ((32 * ts + 16 * (e >> 2) + 4 * g + (e & 3)) * ms + k_off + 16 * db + i16) * ES);
       }
     }
+#pragma unroll
+    for (int f = 0; f < RT; ++f)   // row 2 (RT wave + f) + lane / 32, columns 4 (lane % 32) ..: T, then P
+      rl[f] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     orr, ((2 * (RT * wave + f) + (lane >> 5)) * os + (uint32_t)h * GC_D + 4 * (lane & 31)) * 4, 0, 0));
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -447,32 +465,68 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
   for (int64_t t0 = begin; t0 < end; t0 += C) {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the last chunk's readers are done
     {
+      // an opaque copy of the lane: the addresses below are made here for each
+      // chunk; kept over the loop they cost the registers that are not there
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      if constexpr (NP == 1) {
 #pragma unroll
-      for (int f = 0; f < FK; ++f) {
-        bf16x8 a[NP], q[NP];
-        rk[f].parts(a);
-        rq[f].parts(q);
+        for (int f = 0; f < FK; ++f) {
+          const int t = 8 * wave + 4 * f + (ln >> 4), c = ln & 15;   // token, chunk of 8 dims
+          const int step = c >> 2, hh = (c >> 1) & 1;
+          const u32x4 kw = __builtin_bit_cast(u32x4, rk[f].v), qw = __builtin_bit_cast(u32x4, rq[f].v);
 #pragma unroll
-        for (int n = 0; n < NP; ++n) {
-          *frag(L::KF, (wave * FK + f) * NP + n) = a[n];
-          *frag(L::QF, (wave * FK + f) * NP + n) = q[n];
+          for (int half = 0; half < 2; ++half) {   // dims 4 half .. of the chunk: lane group 2 (c % 2) + half
+            const int at = ((t >> 4) * 4 + step) * 1024 + gc_slot(2 * (c & 1) + half, t & 15, x_k(step)) + 8 * hh;
+            *reinterpret_cast<u32x2*>(smem + L::KF + at) = (u32x2){kw[2 * half], kw[2 * half + 1]};
+            *reinterpret_cast<u32x2*>(smem + L::QF + at) = (u32x2){qw[2 * half], qw[2 * half + 1]};
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {   // K^T: token t is term 4 h + r of lane group (t % 16) / 4
+            const int db = c >> 1, i = 8 * (c & 1) + e;
+            *reinterpret_cast<bf16*>(smem + L::KT + (db * TS + (t >> 5)) * 1024 +
+                                     gc_slot((t & 15) >> 2, i, x_t(db)) + (4 * ((t >> 4) & 1) + (t & 3)) * 2) = rk[f].v[e];
+          }
+        }
+      } else {
+#pragma unroll
+        for (int f = 0; f < FK; ++f) {
+          const int id = wave * FK + f;
+          bf16x8 a[NP], q[NP];
+          rk[f].parts(a);
+          rq[f].parts(q);
+#pragma unroll
+          for (int n = 0; n < NP; ++n) {
+            *frag(L::KF, id * NP + n, x_k(id & 3)) = a[n];
+            *frag(L::QF, id * NP + n, x_k(id & 3)) = q[n];
+          }
+        }
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+          const int id = wave * FT + f;
+          bf16x8 a[NP];
+          rt[f].parts(a);
+#pragma unroll
+          for (int n = 0; n < NP; ++n) *frag(L::KT, id * NP + n, x_t(id / TS)) = a[n];
         }
       }
 #pragma unroll
-      for (int f = 0; f < FT; ++f) {
-        bf16x8 a[NP];
-        rt[f].parts(a);
-#pragma unroll
-        for (int n = 0; n < NP; ++n) *frag(L::KT, (wave * FT + f) * NP + n) = a[n];
-      }
-      if (wave < FP) {
-        bf16x8 a[3], q[3];
-        gc_split<3>(rT, a);
-        gc_split<3>(rP, q);
+      for (int f = 0; f < RT; ++f) {
+        const int t = 2 * (RT * wave + f) + (ln >> 5), c = ln & 15;   // row, chunk of 4 columns of T or P
+        const int ts = c >> 3, hh = (c >> 2) & 1, grp = c & 3;
+        if (TS == 1 && ts) continue;   // f32 chunks have 32 columns
+        f32x2 r0 = {rl[f][0], rl[f][1]}, r1 = {rl[f][2], rl[f][3]};
+        char* at = smem + ((ln & 16) ? L::PF : L::TF) + ((t >> 4) * TS + ts) * 3 * 1024 +
+                   gc_slot(grp, t & 15, x_l(grp, ts)) + 8 * hh;
 #pragma unroll
         for (int n = 0; n < 3; ++n) {
-          *frag(L::TF, wave * 3 + n) = a[n];
-          *frag(L::PF, wave * 3 + n) = q[n];
+          const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r0, bf16x2));
+          const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r1, bf16x2));
+          *reinterpret_cast<u32x2*>(at + n * 1024) = (u32x2){u, w};
+          r0[0] -= __builtin_bit_cast(float, u << 16);
+          r0[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+          r1[0] -= __builtin_bit_cast(float, w << 16);
+          r1[1] -= __builtin_bit_cast(float, w & 0xffff0000u);
         }
       }
       if (wave == GC_WAVES - 1) {
@@ -514,8 +568,8 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
           bf16x8 a[NP], q[NP];
 #pragma unroll
           for (int n = 0; n < NP; ++n) {
-            a[n] = *frag(L::KF, (rb * 4 + s) * NP + n);
-            q[n] = *frag(L::QF, (rb * 4 + s) * NP + n);
+            a[n] = *frag(L::KF, (rb * 4 + s) * NP + n, x_k(s));
+            q[n] = *frag(L::QF, (rb * 4 + s) * NP + n, x_k(s));
           }
           gc_mm<NP, 3>(a, sp[s], kh_, kl);
           gc_mm<NP, 3>(q, sp[s], qh, ql);
@@ -544,7 +598,7 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
         for (int ts = 0; ts <= rb / 2; ++ts) {
           bf16x8 a[3];
 #pragma unroll
-          for (int n = 0; n < 3; ++n) a[n] = *frag(base, (rb * TS + ts) * 3 + n);
+          for (int n = 0; n < 3; ++n) a[n] = *frag(base, (rb * TS + ts) * 3 + n, x_l(g, ts));
           gc_mm<3, 3>(a, up[ts], m[rb], lo);
         }
         m[rb] += lo;
@@ -580,7 +634,7 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
       for (int ts = 0; ts < TS; ++ts) {
         bf16x8 a[NP];
 #pragma unroll
-        for (int n = 0; n < NP; ++n) a[n] = *frag(L::KT, (db * TS + ts) * NP + n);
+        for (int n = 0; n < NP; ++n) a[n] = *frag(L::KT, (db * TS + ts) * NP + n, x_t(db));
         gc_mm<NP, 3>(a, up[ts], S[db], lo);
       }
       S[db] += lo;
