@@ -72,14 +72,8 @@ template <> struct PvType<bf16, false> { typedef bf16 T; };
 // Column of a 4-key group inside a V^T row. bf16: within 16 keys, swap key
 // bits 2 and 3, so lane-half h of the PV product reads its 8 keys
 // {8a + 4h + b} (a, b the S^T accumulator's row split) as one 16-byte chunk.
-// f32: within 32 keys, key 8a + 4h + b goes to 16h + 4a + b.
-template <typename E>
 __device__ __forceinline__ int vcol(int key4) {
-  if constexpr (sizeof(E) == 2) {
-    return (key4 & ~15) | ((key4 & 4) << 1) | ((key4 & 8) >> 1);
-  } else {
-    return (key4 & ~31) | ((key4 & 4) << 2) | ((key4 & 24) >> 1);
-  }
+  return (key4 & ~15) | ((key4 & 4) << 1) | ((key4 & 8) >> 1);
 }
 
 // Four f32 values as three bf16 parts each (8 bytes a part).
@@ -268,8 +262,8 @@ __global__ __launch_bounds__(NW * 64, D <= 64 ? 2 : 1) void attn_fwd_kernel(Attn
       const int id = tid + i * NT;
       if (NVU % NT == 0 || id < NVU) {
         const int g = id / CHK, c = id % CHK;
-        const int col = vcol<E>(4 * g);  // key column of this 4-key group
         if constexpr (ES == 2) {
+          const int col = vcol(4 * g);  // key column of this 4-key group
           // 4 keys x 8 d (bf16) -> for each d, 4 consecutive keys (8 bytes)
 #pragma unroll
           for (int e = 0; e < 8; ++e) {

@@ -354,8 +354,8 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnChunkParams p) {
 // rows (a load of 16 bytes per lane from 16 rows runs at a quarter of the rate
 // of one from 4), so its lanes write one or two rows of many fragments. Against
 // loads in operand order: gdn_chunk_rule 219 -> 197 us at 16 texts of 80 to
-// 1,453 tokens, 16 heads, bf16. f32 loads K and Q in operand order still: their
-// three parts a value leave no registers for a second layout.
+// 1,453 tokens, 16 heads, bf16. f32 still loads K, Q and K^T in operand order;
+// whole rows were not tried there.
 __device__ __forceinline__ int gc_slot(int g, int i, int x) { return (16 * g + (i ^ x)) * 16; }
 template <typename T>
 struct GcLds {
