@@ -85,7 +85,7 @@ constexpr int64_t OWN_GEMM_ROWS = 464;
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct Layout {
-  size_t ids, pos, cu, resid, x, a, b, hf, xf, sched, gemm, total;
+  size_t ids, pos, cu, resid, x, a, b, sched, gemm, total;
   int64_t a_w, b_w;  // row widths (elements) of the two activation buffers
 };
 
@@ -96,10 +96,13 @@ int32_t longest_text(int32_t n_texts, const int32_t* cu) {
 }
 
 // Whether a batch's layers run on the kernels for a few token rows (they take
-// P and V of the attention in f16, which INL_ATTN_PV_BF16 forbids).
-bool is_few(const inl_qwen3_config& c, int64_t n, int32_t longest) {
+// P and V of the attention in f16, which INL_ATTN_PV_BF16 forbids). Their
+// fragments lie in the workspace that hipBLASLt, unused on this path, would
+// get: a workspace of some size takes every smaller batch, on either path.
+bool is_few(const inl_qwen3_config& c, int64_t n, int32_t longest, int64_t x_width, size_t gemm_bytes) {
   return c.attn_flags == 0 &&
-         few_fits(c.dtype, n, longest, c.hidden, c.heads, c.kv_heads, c.head_dim, c.intermediate);
+         few_fits(c.dtype, n, longest, c.hidden, c.heads, c.kv_heads, c.head_dim, c.intermediate) &&
+         up256(few_h_bytes(n, c.hidden)) + few_x_bytes(c.dtype, n, x_width) <= gemm_bytes;
 }
 
 int layout(const inl_qwen3* e, int32_t n_texts, const int32_t* cu, Layout* L) {
@@ -118,9 +121,6 @@ int layout(const inl_qwen3* e, int32_t n_texts, const int32_t* cu, Layout* L) {
   L->x = take((size_t)n * c.hidden * es);
   L->a = take((size_t)n * L->a_w * es);
   L->b = take((size_t)n * L->b_w * es);
-  const bool few = is_few(c, n, longest_text(n_texts, cu));
-  L->hf = take(few ? few_h_bytes(n, c.hidden) : 0);
-  L->xf = take(few ? few_x_bytes(c.dtype, n, L->b_w) : 0);
   inl_attn_desc d{};
   d.n_texts = n_texts;
   d.cu_seqlens_host = cu;
@@ -358,12 +358,12 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
   char* B = ws + L.b;
   void* gws = ws + L.gemm;
   const int32_t longest = longest_text(n_texts, cu);
-  const bool few = is_few(c, n, longest);
-  char* hf = ws + L.hf;
-  char* xf = ws + L.xf;
   size_t gws_bytes = 0;
   rc = inl_linear_workspace_size(&gws_bytes);
   if (rc) return rc;
+  const bool few = is_few(c, n, longest, L.b_w, gws_bytes);
+  char* hf = (char*)gws;
+  char* xf = hf + up256(few_h_bytes(n, c.hidden));
 
   int dev = 0, cus = 0;
   INL_HIP_TRY(hipGetDevice(&dev));

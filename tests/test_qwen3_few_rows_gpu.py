@@ -51,6 +51,20 @@ def test_few_rows_against_oracle(shape, lengths, dtype, cuda, inl):
     enc.close()
 
 
+# A caller may size one workspace for its largest batch: a smaller batch needs
+# no more of it, also where it moves to the few-row kernels.
+@pytest.mark.parametrize("dtype,rows", [("f32", 64), ("bf16", 128)])
+def test_few_rows_need_no_larger_workspace(dtype, rows, cuda, inl):
+    import torch
+    cfg = oq.Qwen3Config(vocab=512, layers=1)
+    td = torch.float32 if dtype == "f32" else torch.bfloat16
+    wd = {k: torch.from_numpy(np.ascontiguousarray(v)).to(cuda).to(td) for k, v in oq.random_weights(cfg, seed=13).items()}
+    enc = inl.Qwen3Encoder(cfg, wd, max_positions=512)
+    sizes = [enc.workspace_bytes([0, n]) for n in (1, rows - 1, rows, rows + 1)]
+    enc.close()
+    assert sizes == sorted(sizes)
+
+
 # f32 batches above 464 rows run on the library's own f32 GEMM: row counts at
 # the edges of its 128-row tiles and of the path, and widths with other part
 # counts. The tolerance of the general path.
