@@ -289,3 +289,25 @@ def test_chunked_rule_matches_recurrence(case, cuda, inl):
     err = np.abs(got - ref).max() / np.abs(ref).max()
     print(f"chunked rule: max error {err:.3g} of the largest value", flush=True)
     assert err <= 5e-6
+
+
+# Rows that start 8 (bf16) or 16 (f32) bytes past a multiple of 16 or 32, with
+# NaN between them: the chunks load whole rows 16 bytes at a time. The bound of
+# the test above.
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_chunked_rule_strided_rows(dtype, cuda, inl):
+    import torch
+    nk, nv, lens, dk = 1, 2, [63, 65, 7], 128
+    rng = np.random.default_rng(5)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n, width = int(cu[-1]), (2 * nk + nv) * dk
+    mixed = og._r(rng.standard_normal((n, width)).astype(np.float32), dtype)
+    g = (-0.2 * rng.uniform(0, 1, (n, nv))).astype(np.float32)
+    beta = rng.uniform(0, 1, (n, nv)).astype(np.float32)
+    rows = torch.full((n, width + 12), float("nan"), dtype=_tdtype(torch, dtype), device=cuda)[:, 4:4 + width]
+    rows.copy_(_t(torch, mixed, cuda, _tdtype(torch, dtype)))
+    print(f"case=gdn_chunked_rule_strided {dtype}", flush=True)
+    got = inl.gdn_rule(rows, cu.tolist(), nk, nv, dk, dk, _t(torch, g, cuda, torch.float32),
+                       _t(torch, beta, cuda, torch.float32)).cpu().numpy()
+    ref = og.rule_packed(mixed, cu, nk, nv, dk, dk, g.astype(np.float64), beta.astype(np.float64))
+    assert np.abs(got - ref).max() / np.abs(ref).max() <= 5e-6
