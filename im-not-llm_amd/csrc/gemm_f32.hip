@@ -9,7 +9,8 @@
 // MFMA, the leading ones and the small ones apart, so that a small product
 // rounds at its own size. Against f64 the error is below that of an f32 MFMA
 // chain (k / 16 roundings instead of k / 4): a 28-layer encode of 800 rows is
-// 4.9e-7 off, with f32 MFMA GEMMs it was 1.7e-6.
+// 4.9e-7 off, with f32 MFMA GEMMs it was 1.7e-6. An infinity (or a value that
+// rounds to one in bf16, above 3.39e38) gives NaN: its remainder is inf - inf.
 //
 // Kernel: 128 x 128 tiles, 8 waves as 2 (w rows) x 4 (x rows), each 64 x 32 =
 // 2 blocks of v_mfma_f32_32x32x16_bf16. A stage of 32 k goes from memory to

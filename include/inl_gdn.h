@@ -63,9 +63,12 @@ int inl_gdn_gates_fwd(int64_t n_tokens, int32_t value_heads, int32_t dtype,
  * mixed: [n_tokens, 2 nk dk + nv dv] in `dtype` (the convolution's output:
  * q heads, k heads, v heads); g, beta: f32 [n_tokens, nv] with `gate_stride`;
  * out: f32 [n_tokens, nv, dv] with `out_stride` elements between tokens.
- * nv a multiple of nk; 1 <= dk, dv <= 128. The state stays in registers,
- * f32, with fused multiply-adds (the reference's kernel rounds each product
- * and sum; the difference is rounding only). */
+ * nv a multiple of nk; 1 <= dk, dv <= 128. The state stays in registers, f32
+ * (the reference's kernel rounds each product and sum; the difference is
+ * rounding only). With dk = dv = 128, aligned rows and 40 or more tokens per
+ * text on average the tokens run in chunks on the matrix cores, at the same
+ * accuracy; `out` holds intermediate values until the call is done, and an
+ * inf or NaN in a token's row may reach earlier tokens of its chunk. */
 int inl_gdn_rule_fwd(int64_t n_tokens, int32_t n_texts, const int32_t* cu_seqlens,
                      int32_t key_heads, int32_t value_heads, int32_t key_dim,
                      int32_t value_dim, int32_t dtype, const void* mixed,
