@@ -31,9 +31,10 @@
 // add up to the f32 value), of whose nine products the six above 2^-27 are
 // summed in f32 by the MFMAs. bf16 K and Q are taken raw, as the one exact
 // part they are (three products), and their norms scale rows of the results.
-// The running sum of g is kept in f64, so that e^(c_i - c_j) is exact to f32
-// however far the sum has run. Against the f64 recurrence the error is no
-// larger than the per-token kernel's.
+// The running sum of g is kept in f64 and takes no g below -1,000 (e^g is 0 in
+// f32 from -104 on): it stays within 64,000 of zero, where an ulp is 7e-12, so
+// that e^(c_i - c_j) is exact to f32 after any reset, -inf included. Against
+// the f64 recurrence the error is no larger than the per-token kernel's.
 //
 // An MFMA contraction of 32 takes its terms in any order that both operands
 // share. Here lane group g = lane / 16, element e = 4 h + r holds term 16 h +
@@ -236,7 +237,8 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnChunkParams p) {
     return hi;
   };
   const int64_t q_off = (int64_t)kh * GC_D, k_off = (int64_t)(p.nk + kh) * GC_D;
-  const float gv = lane < C ? gc_load_f32(gr, (uint32_t)(lane * p.gs + h) * 4) : 0.f;
+  float gv = lane < C ? gc_load_f32(gr, (uint32_t)(lane * p.gs + h) * 4) : 0.f;
+  gv = gv < -1000.f ? -1000.f : gv;   // (a NaN stays)
   const float bv = lane < C ? gc_load_f32(br, (uint32_t)(lane * p.gs + h) * 4) : 0.f;
   bf16x8 kf[RB][4][NP];
 #pragma unroll

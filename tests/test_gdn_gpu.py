@@ -291,6 +291,33 @@ def test_chunked_rule_matches_recurrence(case, cuda, inl):
     assert err <= 5e-6
 
 
+# Gates that reset the state: e^g is 0 in f32 for all of these, whatever their
+# size, at the first, an inner and the last token of a chunk (64 tokens in bf16,
+# 32 in f32), twice in one chunk, and at a text's first token. What follows a
+# reset depends on the small gates after it alone. The bound of the test above.
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("reset", [-200.0, -1e9, -1e12, -1e15, float(np.finfo(np.float32).min), -np.inf])
+def test_chunked_rule_resets(reset, dtype, cuda, inl):
+    import torch
+    nk, nv, lens, dk = 1, 4, [150, 40, 97], 128
+    rng = np.random.default_rng(9)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(cu[-1])
+    mixed = og._r(rng.standard_normal((n, (2 * nk + nv) * dk)).astype(np.float32), dtype)
+    g = (-0.05 * rng.uniform(0, 1, (n, nv))).astype(np.float32)
+    g[[0, 31, 32, 63, 64, 80, 85, 127, 128, 150, 189, 190, 286], 0] = reset
+    g[[20, 170, 200], 1] = reset
+    g[149, 2] = reset   # head 3: none
+    beta = rng.uniform(0, 1, (n, nv)).astype(np.float32)
+    print(f"case=gdn_chunked_rule_resets {reset} {dtype}", flush=True)
+    got = inl.gdn_rule(_t(torch, mixed, cuda, _tdtype(torch, dtype)), cu.tolist(), nk, nv, dk, dk,
+                       _t(torch, g, cuda, torch.float32), _t(torch, beta, cuda, torch.float32)).cpu().numpy()
+    ref = og.rule_packed(mixed, cu, nk, nv, dk, dk, g.astype(np.float64), beta.astype(np.float64))
+    err = np.abs(got - ref).max(axis=(0, 2)) / np.abs(ref).max(axis=(0, 2))
+    print(f"chunked rule: max error {err} of each head's largest value", flush=True)
+    assert (err <= 5e-6).all()
+
+
 # Rows that start 8 (bf16) or 16 (f32) bytes past a multiple of 16 or 32, with
 # NaN between them: the chunks load whole rows 16 bytes at a time. The bound of
 # the test above.
