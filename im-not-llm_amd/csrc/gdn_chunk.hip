@@ -15,8 +15,11 @@
 // Measured against the per-token kernel, rule alone, 16 heads, bf16: 16 texts
 // of 80 to 1,453 tokens 861 -> 243 us, 16 texts of 2,048 1,216 -> 462 us.
 //
-// Non-finite values: 0 times inf is NaN in a product, so an inf or NaN in a
-// token's row may reach earlier tokens of its own chunk and head as well.
+// What a product cannot do: 0 times inf or NaN is NaN, so a token's inf or NaN
+// would reach earlier tokens of its chunk, and unnormalised K and Q overflow
+// where k / |k| does not. Each of these leaves a chunk's results not finite, so a
+// wave that finds such results takes its columns from that chunk's first token on
+// by the recurrence itself, once its loop is over (S waits in its registers).
 //
 // Two kernels. gdn_chunk_prep computes T and P of every chunk of every text
 // at once (one wave per chunk and head) and leaves them in the rows of `out`
@@ -459,6 +462,71 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
   for (int i = 0; i < 8; ++i) S[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float* vec = reinterpret_cast<float*>(smem + L::VEC);
 
+  // The rows of the chunk at t0 by the recurrence itself, for this wave's 16
+  // columns: lane (g, i16) holds rows 16 b + 4 g .. + 3 of its column.
+  auto walk = [&](int64_t t0) __attribute__((always_inline)) {
+    const int rows = (int)min((int64_t)C, end - t0);
+    const __amdgpu_buffer_rsrc_t mr = gc_rows_of(p.mixed, t0, p.ms, rows, width, ES);
+    const __amdgpu_buffer_rsrc_t orr = gc_rows_of(p.out, t0, p.os, rows, (int64_t)p.nv * GC_D, 4);
+    const __amdgpu_buffer_rsrc_t gr = gc_rows_of(p.g, t0, p.gs, rows, p.nv, 4);
+    const __amdgpu_buffer_rsrc_t br = gc_rows_of(p.beta, t0, p.gs, rows, p.nv, 4);
+    // a token's values, loaded while the one before it is worked on
+    Raw<T> kr[4], qr[4];
+    float dec, bet, vt;
+    auto load_row = [&](Raw<T> (&x)[4], uint32_t off, int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) gc_load<T>(x[b], mr, (t * ms + off + 32 * b + 4 * g) * ES);
+    };
+    auto load_rest = [&](int t) __attribute__((always_inline)) {
+      dec = gc_load_f32(gr, (uint32_t)(t * p.gs + h) * 4);
+      bet = gc_load_f32(br, (uint32_t)(t * p.gs + h) * 4);
+      vt = (float)load_t(mr, (t * ms + v_off) * ES);
+    };
+    f32x4 x[8];   // 32 of a row's 128 values, times 1 / sqrt(|row|^2 + 1e-6)
+    auto normed = [&](const Raw<T> (&r)[4]) __attribute__((always_inline)) {
+      float ss = 0.f;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) ss += r[b].squares();
+      const float inv = 1.0f / sqrtf(gc_rows4(ss) + 1e-6f);
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[2 * b + (e >> 2)][e & 3] = (float)r[b].v[e] * inv;
+    };
+    auto dot_s = [&]() __attribute__((always_inline)) {
+      float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[r] = __builtin_fmaf(S[b][r], x[b][r], s[r]);
+      return gc_rows4((s[0] + s[1]) + (s[2] + s[3]));
+    };
+    load_row(kr, k_off, 0);
+    load_row(qr, q_off, 0);
+    load_rest(0);
+#pragma nounroll
+    for (int t = 0; t < rows; ++t) {
+      normed(kr);
+      load_row(kr, k_off, t + 1);
+      const float d = expf(dec);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) S[b] *= d;
+      const float u = (vt - dot_s()) * bet;
+      load_rest(t + 1);
+#pragma unroll
+      for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[b][r] = __builtin_fmaf(x[b][r], u, S[b][r]);
+      normed(qr);
+      load_row(qr, q_off, t + 1);
+      const float o = dot_s() * (1.0f / sqrtf((float)GC_D));
+      if (g == 0)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), orr,
+                                              (t * os + (uint32_t)h * GC_D + 16 * wave + i16) * 4, 0, 0);
+    }
+  };
+  int64_t by_token = end;   // the recurrence takes over at this token
+
   // The two waves of a SIMD leave each barrier together; with equal priority
   // both split (VALU), then both multiply. Favouring one lets it run ahead into
   // its MFMAs while the other splits.
@@ -546,6 +614,7 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
       for (int r = 0; r < 4; ++r) v[rb][r] = (float)rv[rb][r];
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (t0 + C < end) fetch(t0 + C);
+    if (by_token < end) continue;
 
     const float eall = vec[3 * C];
     auto scale = [&](int which, int rb) __attribute__((always_inline)) {
@@ -612,6 +681,15 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
     lower(L::TF, u);
     split_rows(u);
     lower(L::PF, o);
+    float nan = 0.f;   // unless a result is not finite
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) nan = __builtin_fmaf(o[rb][r], 0.f, nan);
+    if (__any(nan != nan)) {
+      by_token = t0;
+      continue;
+    }
     {
       const int rows = (int)min((int64_t)C, end - t0);
       const __amdgpu_buffer_rsrc_t orr = gc_rows_of(p.out, t0, p.os, rows, (int64_t)p.nv * GC_D, 4);
@@ -642,6 +720,7 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
       S[db] += lo;
     }
   }
+  for (int64_t t0 = by_token; t0 < end; t0 += C) walk(t0);
 }
 
 template <typename T>

@@ -318,6 +318,77 @@ def test_chunked_rule_resets(reset, dtype, cuda, inl):
     assert (err <= 5e-6).all()
 
 
+# Values that the chunked form's products cannot take. Infinities and NaN reach
+# what they reach in the recurrence (a value: its column from its token on; a
+# key, gate or beta: all columns from its token on; a query: its token), earlier
+# tokens and other texts not at all. Large finite values, gates above 0 and betas
+# outside [0, 2] give the recurrence's results, within the bound above of the
+# largest that a column's outputs, or a tenth of its values (what a query reads
+# of the state: q . k / sqrt(dk)), have been so far.
+_F32_MIN = float(np.finfo(np.float32).min)
+ODD_CASES = [("v", np.nan), ("v", np.inf), ("v", _F32_MIN), ("v", 1e30), ("k", np.nan), ("k", -np.inf), ("k", 1e15),
+             ("q", np.nan), ("q", np.inf), ("q", 1e15), ("g", np.nan), ("g", np.inf), ("g", 0.4), ("g", 2.0),
+             ("beta", np.nan), ("beta", -np.inf), ("beta", 3.0), ("beta", -1.0)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("where,value", ODD_CASES)
+def test_chunked_rule_odd_values(where, value, dtype, cuda, inl):
+    import torch
+    nk, nv, lens, dk = 1, 2, [150, 90, 70], 128
+    rng = np.random.default_rng(10)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(cu[-1])
+    mixed = rng.standard_normal((n, (2 * nk + nv) * dk)).astype(np.float32)
+    g = (-0.05 * rng.uniform(0, 1, (n, nv))).astype(np.float32)
+    beta = rng.uniform(0, 1, (n, nv)).astype(np.float32)
+    col = {"q": 5, "k": dk + 5, "v": 2 * dk + 5}
+    # inside a chunk, and the last token of two texts; text 2 has none (two lowest values would overflow the state)
+    at = (17, 100, 149, 239) if value != _F32_MIN else (100, 239)
+    for t in at:
+        if where in col:
+            mixed[t, col[where]] = value
+        else:
+            (g if where == "g" else beta)[t, 0] = value
+    mixed = np.maximum(og._r(mixed, dtype), np.float32(_F32_MIN if dtype == "f32" else -3.3895e38))
+    if value == -np.inf and where in col:
+        mixed[at, col[where]] = value
+    print(f"case=gdn_chunked_rule_odd {where}={value} {dtype}", flush=True)
+    got = inl.gdn_rule(_t(torch, mixed, cuda, _tdtype(torch, dtype)), cu.tolist(), nk, nv, dk, dk,
+                       _t(torch, g, cuda, torch.float32), _t(torch, beta, cuda, torch.float32)).cpu().numpy()
+    with np.errstate(all="ignore"):
+        ref = og.rule_packed(mixed, cu, nk, nv, dk, dk, g.astype(np.float64), beta.astype(np.float64))
+    finite = np.isfinite(ref)
+    assert (np.isfinite(got) == finite).all(), f"{(np.isfinite(got) != finite).sum()} values differ in being finite"
+    ref, got = np.where(finite, ref, 0), np.where(finite, got, 0).astype(np.float64)
+    v = np.abs(mixed[:, 2 * nk * dk:].reshape(n, nv, dk).astype(np.float64))
+    size = np.maximum(np.abs(ref), 0.1 * np.where(np.isfinite(v), v, 0))
+    for a, e in zip(cu[:-1], cu[1:]):
+        held = np.maximum(np.maximum.accumulate(size[a:e], axis=0), 1.0)
+        err = (np.abs(got[a:e] - ref[a:e]) / held).max()
+        print(f"rows {a}-{e}: max error {err:.3g} of the largest value so far", flush=True)
+        assert err <= 5e-6
+
+
+# Positive gates: the state grows by e^0.2 a token, past the size up to which it
+# enters products (10^20, after some 230 tokens). The bound of the test above.
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_chunked_rule_growing_state(dtype, cuda, inl):
+    import torch
+    n, dk = 330, 128
+    rng = np.random.default_rng(11)
+    mixed = og._r(rng.standard_normal((n, 3 * dk)).astype(np.float32), dtype)
+    g = np.full((n, 1), 0.2, np.float32)
+    beta = rng.uniform(0, 1, (n, 1)).astype(np.float32)
+    print(f"case=gdn_chunked_rule_growing {dtype}", flush=True)
+    got = inl.gdn_rule(_t(torch, mixed, cuda, _tdtype(torch, dtype)), [0, n], 1, 1, dk, dk,
+                       _t(torch, g, cuda, torch.float32), _t(torch, beta, cuda, torch.float32)).cpu().numpy()
+    ref = og.rule_packed(mixed, [0, n], 1, 1, dk, dk, g.astype(np.float64), beta.astype(np.float64))
+    err = (np.abs(got - ref) / np.maximum(np.maximum.accumulate(np.abs(ref), axis=0), 1.0)).max()
+    print(f"max error {err:.3g} of the largest value so far, largest {np.abs(ref).max():.3g}", flush=True)
+    assert np.abs(ref).max() > 1e22 and err <= 5e-6
+
+
 # Rows that start 8 (bf16) or 16 (f32) bytes past a multiple of 16 or 32, with
 # NaN between them: the chunks load whole rows 16 bytes at a time. The bound of
 # the test above.
