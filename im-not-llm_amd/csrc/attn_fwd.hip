@@ -44,9 +44,13 @@
 // once per workgroup, while they are staged; the planes of one tile fill LDS
 // (96 KiB at head_dim 128), so the next tile waits in registers. Against
 // v_mfma_f32_32x32x2_f32: 32 passages, 8,110 tokens, 16 / 8 heads of 128
-// causal 312 -> 222 us, error against f64 3.0e-7 -> 1.3e-7. An infinity (or a
-// value that rounds to one in bf16, above 3.39e38) gives NaN: its remainder is
-// inf - inf.
+// causal 312 -> 222 us, error against f64 3.0e-7 -> 1.3e-7. An infinity has no
+// such parts (nor has a value above 3.39e38, which rounds to one: the remainder
+// is inf - inf), and among the products of very large values the small ones may
+// overflow to the other sign: each of these leaves NaN in the rows it reaches. A
+// wave that ends with a NaN does its rows again, one key after another with f32
+// FMAs. Below 2^-110 the last part runs out of exponents: the error of a value
+// is then up to 2^-134.
 
 #include <algorithm>
 #include <cmath>
@@ -120,7 +124,8 @@ __device__ __forceinline__ int frag_at(int frag, int row, int hf, int x) {
 
 // (head_dim 64: two waves per SIMD, 256 registers each. In f32 the split
 // otherwise takes 337, and the short units of a local band then run one
-// workgroup per CU: 106 against 74 us on 16 texts of up to 1,000.)
+// workgroup per CU: 106 against 74 us on 16 texts of up to 1,000. 7 registers
+// of it go to scratch, 78 of head_dim 256's 512; none at head_dim 128.)
 template <typename E, int D, int BN, int NW, bool PV16>
 __global__ __launch_bounds__(NW * 64, D <= 64 ? 2 : 1) void attn_fwd_kernel(AttnParams p) {
   typedef typename PvType<E, PV16>::T PT;
@@ -442,33 +447,52 @@ __global__ __launch_bounds__(NW * 64, D <= 64 ? 2 : 1) void attn_fwd_kernel(Attn
         for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) l_i += sacc[kb][r];
-        bf16x8 pk[NKB * 2][3];
-#pragma unroll
-        for (int ks = 0; ks < NKB * 2; ++ks) {
+        auto split_p = [&](int ks, bf16x8 (&o)[3]) __attribute__((always_inline)) {
           f32x4 a, b;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             a[e] = sacc[ks >> 1][8 * (ks & 1) + e];
             b[e] = sacc[ks >> 1][8 * (ks & 1) + 4 + e];
           }
-          split8(a, b, pk[ks]);
-        }
+          split8(a, b, o);
+        };
+        auto pv = [&](int db, int ks, const bf16x8 (&pk)[3], f32x16& lo) __attribute__((always_inline)) {
+          const char* src0 = sV + frag_at(db * NKB * 2 + ks, lq, hf, db & 3);
+          bf16x8 a[3];
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          if (db * 32 < hd) {
-            f32x16 lo;
+          for (int n = 0; n < 3; ++n) a[n] = *reinterpret_cast<const bf16x8*>(src0 + n * 1024);
+          mfma_split(a, pk, oacc[db], lo);
+        };
+        const f32x16 zero = {};
+        if constexpr (NDB <= 2) {   // one step's P at a time: fewer registers than one block's sums at a time
+          f32x16 lo[NDB];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) lo[r] = 0.f;
+          for (int db = 0; db < NDB; ++db) lo[db] = zero;
 #pragma unroll
-            for (int ks = 0; ks < NKB * 2; ++ks) {
-              const char* src0 = sV + frag_at(db * NKB * 2 + ks, lq, hf, db & 3);
-              bf16x8 a[3];
+          for (int ks = 0; ks < NKB * 2; ++ks) {
+            bf16x8 pk[3];
+            split_p(ks, pk);
 #pragma unroll
-              for (int n = 0; n < 3; ++n) a[n] = *reinterpret_cast<const bf16x8*>(src0 + n * 1024);
-              mfma_split(a, pk[ks], oacc[db], lo);
+            for (int db = 0; db < NDB; ++db)
+              if (db * 32 < hd) pv(db, ks, pk, lo[db]);
+          }
+#pragma unroll
+          for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[db][r] += lo[db][r];
+        } else {
+          bf16x8 pk[NKB * 2][3];
+#pragma unroll
+          for (int ks = 0; ks < NKB * 2; ++ks) split_p(ks, pk[ks]);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            if (db * 32 < hd) {
+              f32x16 lo = zero;
+#pragma unroll
+              for (int ks = 0; ks < NKB * 2; ++ks) pv(db, ks, pk[ks], lo);
+#pragma unroll
+              for (int r = 0; r < 16; ++r) oacc[db][r] += lo[r];
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) oacc[db][r] += lo[r];
           }
         }
       }
@@ -477,6 +501,62 @@ __global__ __launch_bounds__(NW * 64, D <= 64 ? 2 : 1) void attn_fwd_kernel(Attn
     if constexpr (ES == 4) __syncthreads();   // every wave has read the one tile LDS holds
     if (more) store_tile(buf ^ 1);
     __syncthreads();
+  }
+
+  // ---- f32: rows with a NaN again, key by key ----
+  // A lane holds half of its query's dims in O^T's own layout, K and V rows are
+  // the same for all lanes.
+  if constexpr (ES == 4) {
+    float nan = l_i;   // NaN if a result is (or an infinity)
+#pragma unroll
+    for (int i = 0; i < NDB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nan = __builtin_fmaf(oacc[i][r], 0.f, nan);
+    if (__any(nan != nan)) {
+#pragma unroll
+      for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
+      m_i = -INFINITY;
+      l_i = 0.f;
+      // (from an opaque row: the address is not kept in registers over the loop above)
+      int row = qvalid ? qrow : 0;
+      asm volatile("" : "+v"(row));
+      const char* qp0 = p.q + ((int64_t)(seg + row) * p.q_stride + (int64_t)head * hd) * ES;
+      const int k1 = active ? min(khi, hi_t * BN) : 0;
+      for (int key = max(klo, lo_t * BN); key < k1; ++key) {
+        const char* krow = kbase + (int64_t)key * p.k_stride * ES;
+        const char* vrow = vbase + (int64_t)key * p.v_stride * ES;
+        float s = 0.f;
+        for (int c = hf; c * VEC < hd; c += 2) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(krow + c * 16);
+          const f32x4 b = *reinterpret_cast<const f32x4*>(qp0 + c * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s = __builtin_fmaf(a[e], b[e], s);
+        }
+        s = half_sum(s);
+        bool sees = qvalid && (!p.causal || key <= qrow);
+        if (p.window >= 0) sees = sees && abs(qrow - key) <= p.window;
+        if (!sees) s = -INFINITY;
+        const float m_new = fmaxf(m_i, s * c2);
+        const float base = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_i - base);
+        const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(s, c2, -base));
+        m_i = m_new;
+        l_i = l_i * alpha + (hf == 0 ? w : 0.f);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const int d0 = db * 32 + 8 * g + 4 * hf;
+            f32x4 val = {0.f, 0.f, 0.f, 0.f};
+            if (d0 < hd && sees) val = *reinterpret_cast<const f32x4*>(vrow + d0 * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              oacc[db][4 * g + e] = __builtin_fmaf(w, val[e], oacc[db][4 * g + e] * alpha);
+          }
+      }
+    }
   }
 
   // ---- epilogue: O = O^T / l, one query row per lane column ----

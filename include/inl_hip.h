@@ -103,6 +103,11 @@ typedef struct inl_attn_desc {
  * keeps V and P in bf16 (any range, 8x coarser P). */
 #define INL_ATTN_PV_BF16 1
 
+/* f32 inputs: products of three bf16 parts of each value, as accurate as f32
+ * products (values below 2^-110 in magnitude: to an absolute 2^-134). Rows that
+ * an infinity, a NaN, or magnitudes near the end of f32's range reach are done
+ * again by f32 FMAs, slowly, so that a score of -inf keeps weight 0. */
+
 /* f32 descs: a batch too small to fill the GPU (fewer query blocks x head
  * groups than workgroups the GPU holds at once) has its longer query blocks'
  * key ranges split into parts that run as separate workgroups, and a second

@@ -278,3 +278,54 @@ def test_f32_parts_every_head_dim(d, causal, window, cuda, inl):
         r = ref[cu[b]:cu[b + 1]]
         bound = 2e-6 * np.abs(v[cu[b]:cu[b + 1]].cpu().numpy()).max()
         assert np.abs(out[cu[b]:cu[b + 1]] - r).max() <= bound
+
+
+@pytest.mark.parametrize("d", [16, 64, 72, 128, 256])
+@pytest.mark.parametrize("what,value", [("k", -np.inf), ("k", "lowest"), ("k", -1e37), ("v", -3.395e38), ("v", np.inf),
+                                        ("q", 1e20), ("k", np.nan)])
+def test_f32_values_without_parts(what, value, d, cuda, inl):
+    """f32 attention on infinities and on values so large that their bf16 parts
+    do not exist or multiply to infinities of both signs. Keys whose row holds
+    -inf or a huge negative value have weight 0 (q > 0 in that column) and drop
+    out; values show in the outputs that see them. Finite outputs as the f64
+    oracle, within 2e-6 of the largest value that a row's head sees; the others
+    not finite; texts without such values unchanged. Short texts run with a split
+    key range (NO_SPLIT: without)."""
+    import torch
+    lengths = [1, 70, 200, 33]
+    hq, hkv = 4, 2
+    (q, k, v), _ = _inputs(lengths, hq, hkv, d, d + 1, torch.float32, torch, cuda, d ** -0.5)
+    value = float(np.finfo(np.float32).min) if value == "lowest" else value
+    cu = oa.cu_from_lengths(lengths)
+    # none first in a 32-key tile, where it would be the largest score of a split's part
+    keys = [int(cu[1]) + 5, int(cu[1]) + 40, int(cu[2]) + 65, int(cu[2]) + 130]
+    if what == "k":
+        q[..., 3] = q[..., 3].abs() * 0.5 + 0.01
+        if value == value:   # other columns add nothing to an infinite score
+            k[keys] = 0.0
+        k[keys, :, 3] = value
+    elif what == "v":
+        keys = keys[::2]   # one a text: the sum of two overflows, and a weight of 1 + 2^-23 times the lowest
+        v[keys, :, 3] = value
+    else:   # large queries on small keys: scores of order 1
+        q[keys] *= value
+        k /= value
+    host = [t.cpu().numpy().astype(np.float64) for t in (q, k, v)]
+    infinite = np.isinf(host[2])   # reach the rows that see them, nothing else
+    host[2][infinite] = 0.0
+    with np.errstate(all="ignore"):
+        ref = oa.varlen_attention(*host, cu, causal=True, scale=d ** -0.5)
+    finite = np.isfinite(ref)
+    for a, e in zip(cu[:-1], cu[1:]):
+        finite[a:e] &= ~np.repeat(np.logical_or.accumulate(infinite[a:e], axis=0), hq // hkv, axis=1)
+    seen = np.zeros_like(ref)   # largest |v| that a row's head sees
+    top = np.repeat(np.abs(host[2]).max(-1), hq // hkv, axis=1)
+    for a, e in zip(cu[:-1], cu[1:]):
+        seen[a:e] = np.maximum.accumulate(top[a:e], axis=0)[..., None]
+    for flags in (0, inl.ATTN_NO_SPLIT):
+        print(f"case=f32_values {what}={value} d={d} flags={flags}", flush=True)
+        assert finite.any()
+        got = inl.varlen_attention(q, k, v, cu.tolist(), causal=True, flags=flags).cpu().numpy()
+        assert (np.isfinite(got) == finite).all()
+        err = np.abs(np.where(finite, got, 0) - np.where(finite, ref, 0)) / seen
+        assert err.max() <= 2e-6
