@@ -126,8 +126,9 @@ __device__ __forceinline__ int frag_at(int frag, int row, int hf, int x) {
 // otherwise takes 337, and the short units of a local band then run one
 // workgroup per CU: 106 against 74 us on 16 texts of up to 1,000. 7 registers
 // of it go to scratch, 78 of head_dim 256's 512; none at head_dim 128.)
+constexpr int waves_per_simd(int d) { return d <= 64 ? 2 : 1; }
 template <typename E, int D, int BN, int NW, bool PV16>
-__global__ __launch_bounds__(NW * 64, D <= 64 ? 2 : 1) void attn_fwd_kernel(AttnParams p) {
+__global__ __launch_bounds__(NW * 64, waves_per_simd(D)) void attn_fwd_kernel(AttnParams p) {
   typedef typename PvType<E, PV16>::T PT;
   constexpr int NT = NW * 64;
   constexpr int ES = (int)sizeof(E);
@@ -1227,7 +1228,9 @@ void split_key_ranges(const inl_attn_desc* d, std::vector<CostedItem>& tmp, Sche
   if (d->dtype != INL_F32 || (d->flags & INL_ATTN_NO_SPLIT) || tmp.empty()) return;
   const int max_tiles = tmp.front().cost;  // sorted longest first
   if (max_tiles < 2) return;
-  const int64_t resident = (int64_t)device_cus() * std::max(1, kLdsPerCu / std::max(1, s->cfg.lds));
+  // workgroups (one wave per SIMD each) that a CU holds, by LDS and by registers
+  const int per_cu = std::min(kLdsPerCu / std::max(1, s->cfg.lds), waves_per_simd(s->cfg.d));
+  const int64_t resident = (int64_t)device_cus() * std::max(1, per_cu);
   if ((int64_t)tmp.size() * s->n_hg > 16 * resident) return;
   auto est = [&](int c) {
     std::vector<int> parts;

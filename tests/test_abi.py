@@ -343,3 +343,21 @@ def test_small_f32_batches_split_their_key_ranges():
     bad = inl_hip.make_attn_desc(small, 16, 8, 128, causal=True, dtype="f32", flags=4)
     assert inl_hip._ws_size(ctypes.byref(bad), ctypes.byref(n)) != 0
     assert "unknown flags" in inl_hip.last_error()
+
+
+def test_f32_split_counts_the_workgroups_that_fit_a_cu():
+    """The key-range split is planned for the workgroups a GPU holds at once:
+    at head_dim 64 two per CU (registers), although LDS would hold three. 24
+    texts of 341 tokens, 12 heads, radius 64 fill two per CU as they are; 16
+    such texts do not."""
+    import inl_hip
+    n = ctypes.c_size_t()
+
+    def ws(texts, flags=0):
+        cu = list(range(0, 341 * texts + 1, 341))
+        d = inl_hip.make_attn_desc(cu, 12, 12, 64, causal=False, window=64, dtype="f32", flags=flags)
+        assert inl_hip._ws_size(ctypes.byref(d), ctypes.byref(n)) == 0, inl_hip.last_error()
+        return n.value
+
+    assert ws(24) == ws(24, inl_hip.ATTN_NO_SPLIT)
+    assert ws(16) > ws(16, inl_hip.ATTN_NO_SPLIT)
