@@ -9,8 +9,10 @@
 // MFMA, the leading ones and the small ones apart, so that a small product
 // rounds at its own size. Against f64 the error is below that of an f32 MFMA
 // chain (k / 16 roundings instead of k / 4): a 28-layer encode of 800 rows is
-// 4.9e-7 off, with f32 MFMA GEMMs it was 1.7e-6. An infinity (or a value that
-// rounds to one in bf16, above 3.39e38) gives NaN: its remainder is inf - inf.
+// 4.9e-7 off, with f32 MFMA GEMMs it was 1.7e-6. What has no such parts (an
+// infinity, or a value above 3.39e38, which rounds to one in bf16: the remainder
+// is inf - inf) makes every product it enters NaN. A wave that finds a NaN among
+// its results therefore multiplies its block again, on the f32 MFMA.
 //
 // Kernel: 128 x 128 tiles, 8 waves as 2 (w rows) x 4 (x rows), each 64 x 32 =
 // 2 blocks of v_mfma_f32_32x32x16_bf16. A stage of 32 k goes from memory to
@@ -203,6 +205,32 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_f32_kernel(GemmF32Params p) {
     stage(s + 1, 1, r0);
   }
   if (s < stages) stage(s, 0, r1);
+
+  {
+    float s = 0.f;   // NaN if a result is NaN (or infinite)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s = __builtin_fmaf(hi[q][r] + lo[q][r], 0.f, s);
+    if (__any(s != s)) {
+      // lane half hf takes 4 k of each 8, of w row l32 of a block and x row l32
+      const int xrow = wm * 32 + l32;
+      const uint32_t xo = xrow < xrows ? (uint32_t)(xrow * p.xs * 4) + hf * 16 : 0x80000000u;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int wrow = EPI == GF_SWIGLU ? wn * 32 + l32 + q * p.n : (wn * 2 + q) * 32 + l32;
+        const uint32_t wo = (uint32_t)(wrow * p.ws * 4) + hf * 16;
+        hi[q] = lo[q] = zero;
+#pragma nounroll
+        for (int k = 0; k < kp; k += 8) {
+          const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, k * 4, 0));
+          const f32x4 b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo, k * 4, 0));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) hi[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], hi[q], 0, 0, 0);
+        }
+      }
+    }
+  }
 
   // Epilogue: lane holds x row l32 of its wave's 32, w rows 8 g + 4 hf + e of
   // each block. Through LDS (32 rows x 272 bytes per wave), so that a store

@@ -85,3 +85,27 @@ def test_f32_gemm_rows_against_oracle(shape, lengths, cuda, inl):
     ref = oq.encode(w, cfg, ids, cu)
     cos = (got * ref).sum(1) / np.linalg.norm(got, axis=1) / np.linalg.norm(ref, axis=1)
     assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4
+
+
+# A gate row of the lowest f32 value: its products are finite (silu gives -0),
+# but it has no bf16 parts. Within the f32 tolerance of the oracle.
+def test_f32_gemm_lowest_weight(cuda, inl):
+    import torch
+    cfg = oq.Qwen3Config(vocab=64, layers=1, hidden=512, intermediate=256, heads=8, kv_heads=8)
+    w = oq.random_weights(cfg, seed=15)
+    w["embed_tokens.weight"][:, 0] = np.abs(w["embed_tokens.weight"][:, 0]) + 0.01   # x[0] > 0 at the gate
+    w["layers.0.self_attn.o_proj.weight"][0] = 0
+    w["layers.0.post_attention_layernorm.weight"][0] = 0.01
+    gate = w["layers.0.mlp.gate_proj.weight"]
+    gate[[3, 130]] = 0
+    gate[[3, 130], 0] = np.finfo(np.float32).min
+    wd = {k: torch.from_numpy(np.ascontiguousarray(v)).to(cuda) for k, v in w.items()}
+    ids = np.random.default_rng(1).integers(0, cfg.vocab, 700)
+    cu = [0, 300, 700]
+    print("case=f32_gemm lowest weight", flush=True)
+    enc = inl.Qwen3Encoder(cfg, wd, max_positions=512)
+    got = enc.encode(ids, cu).cpu().numpy().astype(np.float64)
+    enc.close()
+    with np.errstate(over="ignore"):
+        ref = oq.encode(w, cfg, ids, cu)
+    assert np.isfinite(ref).all() and np.abs(got - ref).max() <= 1e-6
