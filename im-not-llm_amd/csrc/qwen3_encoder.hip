@@ -54,6 +54,7 @@ struct inl_qwen3 {
   inl_qwen3_config cfg;
   const void* embed = nullptr;
   std::vector<inl_qwen3_layer_weights> layers;
+  bool vec16 = true;                // every layer weight starts on a 16-byte boundary
   float* final_norm_f32 = nullptr;  // device, owned
   float* cos = nullptr;             // device, owned: [max_positions, head_dim / 2]
   float* sin = nullptr;
@@ -98,9 +99,12 @@ int32_t longest_text(int32_t n_texts, const int32_t* cu) {
 // Whether a batch's layers run on the kernels for a few token rows (they take
 // P and V of the attention in f16, which INL_ATTN_PV_BF16 forbids). Their
 // fragments lie in the workspace that hipBLASLt, unused on this path, would
-// get: a workspace of some size takes every smaller batch, on either path.
-bool is_few(const inl_qwen3_config& c, int64_t n, int32_t longest, int64_t x_width, size_t gemm_bytes) {
-  return c.attn_flags == 0 &&
+// get: a workspace of some size takes every smaller batch, on either path. They
+// read all weights 16 bytes at a time; a model whose weights do not start on
+// such boundaries runs the general sequence, which takes or refuses them.
+bool is_few(const inl_qwen3* e, int64_t n, int32_t longest, int64_t x_width, size_t gemm_bytes) {
+  const inl_qwen3_config& c = e->cfg;
+  return e->vec16 && c.attn_flags == 0 &&
          few_fits(c.dtype, n, longest, c.hidden, c.heads, c.kv_heads, c.head_dim, c.intermediate) &&
          up256(few_h_bytes(n, c.hidden)) + few_x_bytes(c.dtype, n, x_width) <= gemm_bytes;
 }
@@ -245,6 +249,10 @@ extern "C" int inl_qwen3_create(const inl_qwen3_config* cfg, const void* embed_t
   e->cfg = *cfg;
   e->embed = embed_tokens;
   e->layers.assign(layers, layers + cfg->layers);
+  for (const inl_qwen3_layer_weights& l : e->layers)
+    for (const void* w : {l.qkv_proj, l.o_proj, l.gate_up_proj, l.down_proj, l.q_norm, l.k_norm, l.input_norm,
+                          l.post_attention_norm})
+      e->vec16 = e->vec16 && ((uintptr_t)w & 15) == 0;
   const int half = cfg->head_dim / 2;
   std::vector<float> c((size_t)cfg->max_positions * half), s(c.size());
   rc = inl_rope_table_host(cfg->head_dim, cfg->rope_theta, cfg->max_positions, 0, c.data(), s.data());
@@ -361,7 +369,7 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
   size_t gws_bytes = 0;
   rc = inl_linear_workspace_size(&gws_bytes);
   if (rc) return rc;
-  const bool few = is_few(c, n, longest, L.b_w, gws_bytes);
+  const bool few = is_few(e, n, longest, L.b_w, gws_bytes);
   char* hf = (char*)gws;
   char* xf = hf + up256(few_h_bytes(n, c.hidden));
 
@@ -418,8 +426,9 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
     return rc;
   }
 
-  // (a projection's parts go to the workspace that hipBLASLt would get)
-  const bool own = !few && dt == INL_F32 && gemm_f32_fits(c.hidden, (int32_t)qkv_w, (int32_t)qd, c.intermediate) &&
+  // (a projection's parts go to the workspace that hipBLASLt would get; the
+  // weights are read 16 bytes at a time, as by the few-row kernels)
+  const bool own = !few && e->vec16 && dt == INL_F32 && gemm_f32_fits(c.hidden, (int32_t)qkv_w, (int32_t)qd, c.intermediate) &&
                    (size_t)n * c.hidden * 4 <= gws_bytes && n > OWN_GEMM_ROWS;
   const int o_parts = own ? gemm_f32_splits(n, c.hidden, (int32_t)qd, cus, gws_bytes) : 1;
   const int d_parts = own ? gemm_f32_splits(n, c.hidden, c.intermediate, cus, gws_bytes) : 1;

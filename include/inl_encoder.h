@@ -159,6 +159,9 @@ typedef struct inl_qwen3_config {
   int32_t attn_flags;     /* INL_ATTN_* (INL_ATTN_PV_BF16 for V beyond fp16) */
 } inl_qwen3_config;
 
+/* Weights of any alignment, except q_norm and k_norm (16 bytes). The kernels for
+ * a few rows and the f32 GEMM need all of a model's layer weights on 16-byte
+ * boundaries; other models run the general sequence. */
 typedef struct inl_qwen3_layer_weights {
   const void* qkv_proj;
   const void* o_proj;         /* [hidden, heads * head_dim] */

@@ -87,6 +87,45 @@ def test_f32_gemm_rows_against_oracle(shape, lengths, cuda, inl):
     assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4
 
 
+# Weights that are slices of a larger buffer, one element off a 16-byte boundary:
+# the few-row and f32-GEMM kernels load 16 bytes at a time, so such a model takes
+# the general sequence, for which unaligned row norms are ordinary and unaligned
+# q/k norms an error. Against the encode of the same weights, aligned, within the
+# sum of both paths' distances from the oracle above.
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows", [17, 500])
+def test_unaligned_weights(rows, dtype, cuda, inl):
+    import torch
+    cfg = oq.Qwen3Config(vocab=512, layers=1)
+    td = torch.float32 if dtype == "f32" else torch.bfloat16
+    wd = {k: torch.from_numpy(np.ascontiguousarray(v)).to(cuda).to(td) for k, v in oq.random_weights(cfg, seed=14).items()}
+    ids = np.random.default_rng(rows).integers(0, cfg.vocab, rows)
+
+    def shifted(name):
+        buf = torch.empty(wd[name].numel() + 1, dtype=td, device=cuda)
+        buf[1:] = wd[name].reshape(-1)
+        view = buf[1:].view(wd[name].shape)
+        assert view.data_ptr() % 16 == view.element_size()
+        return {**wd, name: view}
+
+    def encode(weights):
+        enc = inl.Qwen3Encoder(cfg, weights, max_positions=512)
+        try:
+            return enc.encode(ids, [0, rows]).cpu().numpy()
+        finally:
+            enc.close()
+
+    print(f"case=unaligned weights {dtype} rows={rows}", flush=True)
+    want = encode(wd)
+    for name in ("input_layernorm.weight", "post_attention_layernorm.weight"):
+        got = encode(shifted("layers.0." + name))
+        cos = (got * want).sum(1) / np.linalg.norm(got, axis=1) / np.linalg.norm(want, axis=1)
+        assert cos.min() >= (1 - 2e-5 if dtype == "f32" else 1 - 2e-3)
+    for name in ("q_norm.weight", "k_norm.weight"):
+        with pytest.raises(inl.InlError):
+            encode(shifted("layers.0.self_attn." + name))
+
+
 # A gate row of the lowest f32 value: its products are finite (silu gives -0),
 # but it has no bf16 parts. Within the f32 tolerance of the oracle.
 def test_f32_gemm_lowest_weight(cuda, inl):
