@@ -306,6 +306,11 @@ bool gemm_f32_fits(int32_t hidden, int32_t qkv_rows, int32_t attn_width, int32_t
          (int64_t)GF_BN * std::max(attn_width, intermediate) * 4 < ((int64_t)1 << 31);
 }
 
+bool gemm_f32_pays(int64_t m, int32_t qkv_rows) {
+  const int64_t tiles = (m + GF_BM - 1) / GF_BM * (qkv_rows / GF_BN);
+  return m > 464 && tiles >= 128;
+}
+
 int gemm_f32_splits(int64_t m, int32_t n, int32_t k, int cus, size_t part_bytes) {
   // parts until every CU has a workgroup, while a part keeps 8 stages
   const int64_t tiles = (m + GF_BM - 1) / GF_BM * (n / GF_BN);

@@ -76,13 +76,6 @@ namespace inl {
 
 namespace {
 
-// f32 batches of more rows than this run on the library's own GEMM, smaller
-// ones on hipBLASLt (us per encode of the 0.6B shape, own / hipBLASLt: 400 rows
-// 5,109 / 4,993, 512 rows 5,357 / 6,405, 800 6,986 / 7,811, 1,024 7,505 /
-// 11,350, 2,048 12,408 / 15,582: a 128-row tile's k loop is serial, and few
-// tiles leave CUs idle).
-constexpr int64_t OWN_GEMM_ROWS = 464;
-
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct Layout {
@@ -429,7 +422,7 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
   // (a projection's parts go to the workspace that hipBLASLt would get; the
   // weights are read 16 bytes at a time, as by the few-row kernels)
   const bool own = !few && e->vec16 && dt == INL_F32 && gemm_f32_fits(c.hidden, (int32_t)qkv_w, (int32_t)qd, c.intermediate) &&
-                   (size_t)n * c.hidden * 4 <= gws_bytes && n > OWN_GEMM_ROWS;
+                   (size_t)n * c.hidden * 4 <= gws_bytes && gemm_f32_pays(n, (int32_t)qkv_w);
   const int o_parts = own ? gemm_f32_splits(n, c.hidden, (int32_t)qd, cus, gws_bytes) : 1;
   const int d_parts = own ? gemm_f32_splits(n, c.hidden, c.intermediate, cus, gws_bytes) : 1;
 

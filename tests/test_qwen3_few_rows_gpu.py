@@ -69,7 +69,7 @@ def test_few_rows_need_no_larger_workspace(dtype, rows, cuda, inl):
 # the edges of its 128-row tiles and of the path, and widths with other part
 # counts. The tolerance of the general path.
 @pytest.mark.parametrize("shape,lengths", [("0.6B", [465]), ("0.6B", [200, 312]), ("0.6B", [300, 200, 140, 1]),
-                                           ("group1", [500, 13]), ("group4", [512, 257])])
+                                           ("group1", [500, 13]), ("group4", [512, 257]), ("group1", [500, 200])])
 def test_f32_gemm_rows_against_oracle(shape, lengths, cuda, inl):
     import torch
     cfg = oq.Qwen3Config(vocab=512, layers=2, **SHAPES[shape])
