@@ -448,11 +448,15 @@ extern "C" int inl_qwen3_encode(inl_qwen3* e, int32_t n_texts, const int32_t* cu
     const inl_qwen3_layer_weights& w = e->layers[i];
     if (few) {
       hipStream_t sq = (hipStream_t)stream;
-      const SkinnyNext to_o = skinny_next(dt, w.o_proj, c.hidden, (int32_t)qd, false);
-      const SkinnyNext to_gu = skinny_next(dt, w.gate_up_proj, c.intermediate, c.hidden, true);
-      const SkinnyNext to_down = skinny_next(dt, w.down_proj, c.hidden, c.intermediate, false);
-      const SkinnyNext to_qkv = i + 1 < c.layers
-          ? skinny_next(dt, e->layers[i + 1].qkv_proj, (int32_t)qkv_w, c.hidden, false) : SkinnyNext{};
+      const bool ahead = few_prefetch(dt, n);
+      auto next = [&](const void* w, int32_t rows, int64_t width, bool swiglu) {
+        return ahead ? skinny_next(dt, w, rows, (int32_t)width, swiglu, cus) : SkinnyNext{};
+      };
+      const SkinnyNext to_o = next(w.o_proj, c.hidden, qd, false);
+      const SkinnyNext to_gu = next(w.gate_up_proj, c.intermediate, c.hidden, true);
+      const SkinnyNext to_down = next(w.down_proj, c.hidden, c.intermediate, false);
+      const SkinnyNext to_qkv =
+          i + 1 < c.layers ? next(e->layers[i + 1].qkv_proj, (int32_t)qkv_w, c.hidden, false) : SkinnyNext{};
       rc = skinny_launch(dt, n, (int32_t)qkv_w, c.hidden, hf, w.input_norm, c.eps, w.qkv_proj, SKINNY_STORE, A, L.a_w,
                          nullptr, SkinnyNext{}, sq);
       if (!rc) rc = few_attn(dt, n_texts, n, longest, d_cu, A, L.a_w, c.heads, c.kv_heads, w.q_norm, w.k_norm, c.eps,

@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void skinny_kernel(SkinnyParams p) {
   __shared__ __attribute__((aligned(1024))) char own[SK_WAVES][OWN];
   __shared__ float ssum[SK_WAVES][MB * 16];
   if ((int)blockIdx.x >= p.n / 16) {
-    if (blockIdx.y == 0) prefetch_next(p.next, p.n / 16, gridDim.x);
+    prefetch_next(p.next, p.n / 16, gridDim.x);   // (only launched beside one row of workgroups)
     return;
   }
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void skinny_kernel(SkinnyParams p) {
 }
 
 // Prefetching workgroups beside `own` working ones: the CUs left over.
-int prefetchers(const SkinnyNext& q, int own) { return q.w && own < 256 ? 256 - own : 0; }
+int prefetchers(const SkinnyNext& q, int own) { return q.w && own < q.cus ? q.cus - own : 0; }
 
 // ---- embedding: h[t, :] = f32(table[ids[t], :]), as rows and as fragments ----
 // One workgroup per token row; an id outside [0, vocab) gives a NaN row.
@@ -772,6 +772,8 @@ void by_kind(const SkinnyParams& p, bool norm, int epi, hipStream_t st) {
 }
 
 }  // namespace
+
+bool few_prefetch(int32_t dtype, int64_t n) { return n <= (dtype == INL_BF16 ? 64 : 32); }
 
 bool few_fits(int32_t dtype, int64_t n, int32_t longest, int32_t hidden, int32_t heads, int32_t kv_heads,
               int32_t head_dim, int32_t intermediate) {

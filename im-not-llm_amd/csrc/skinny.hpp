@@ -18,10 +18,11 @@ struct SkinnyNext {
   const char* w = nullptr;   // nullptr: nothing to prefetch
   int64_t bytes = 0, second = 0;
   int32_t consumers = 0;
+  int32_t cus = 0;           // of the device: a workgroup on each that the launch itself leaves idle
 };
-inline SkinnyNext skinny_next(int32_t dtype, const void* w, int32_t n, int32_t k, bool swiglu) {
+inline SkinnyNext skinny_next(int32_t dtype, const void* w, int32_t n, int32_t k, bool swiglu, int32_t cus) {
   const int64_t row = (int64_t)k * dtype_size(dtype);
-  return {(const char*)w, 16 * row, swiglu ? n * row : 0, n / 16};
+  return {(const char*)w, 16 * row, swiglu ? n * row : 0, n / 16, cus};
 }
 
 // y[m, n] from x[m, k] . w[n, k]^T, x in fragments xf. gamma != NULL: xf
@@ -34,9 +35,17 @@ int skinny_launch(int32_t dtype, int64_t m, int32_t n, int32_t k, const void* xf
 // Token rows up to which a layer runs this way. Measured against the general
 // path, us per encode of the 0.6B shape: bf16 897 / 2,066 at 17 rows, 1,184 /
 // 2,205 at 64, 1,719 / 2,154 at 128 (there every projection is two workgroup
-// rows, and 256 rows would be four); f32 1,575 / 2,412 at 17, 2,500 / 2,825 at
+// rows, and 256 rows would be four); f32 1,575 / 2,412 at 17, 2,261 / 2,825 at
 // 64, 3,298 / 2,648 at 128: f32 MFMAs take 16 times as long.
 constexpr int64_t FEW_ROWS_BF16 = 128, FEW_ROWS_F32 = 64;
+
+// Whether the launches prefetch: while one row of workgroups covers all n rows (64
+// in bf16, 32 in f32). The workgroups of a second row would wait behind the
+// prefetchers. us per encode of the 0.6B shape, with / without: bf16 17 rows 914 /
+// 994, 64 rows 1,287 / 1,379, 128 rows (two rows of workgroups) 1,742 / 1,725; f32
+// 8 rows 1,161 / 1,303, 32 rows 1,590 / 1,701, 48 rows (two) 2,415 / 1,983, 64
+// rows (two) 2,710 / 2,261.
+bool few_prefetch(int32_t dtype, int64_t n);
 
 // Whether a batch (n rows, longest text) of a model of this shape can.
 bool few_fits(int32_t dtype, int64_t n, int32_t longest, int32_t hidden, int32_t heads, int32_t kv_heads,
