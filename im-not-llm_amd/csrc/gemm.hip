@@ -553,3 +553,21 @@ extern "C" int inl_gemm_bf16_gated_fwd(int64_t m, int64_t n, int64_t k, const vo
   return gemm_launch(mode == INL_GATE_GEGLU ? EPI_GEGLU : EPI_GELU_MUL, m, n, k, x, x_stride, w, w_stride, mul,
                      mul_stride, out_dtype, y, y_stride, 1.f, 0.f, stream);
 }
+
+extern "C" int inl_gemm_bf16_tile(int32_t mode, int64_t m, int64_t n, int64_t k, int32_t out_dtype, int32_t* x_rows,
+                                  int32_t* w_rows) {
+  using namespace inl;
+  if ((mode != 0 && mode != INL_GATE_GEGLU && mode != INL_GATE_GELU_MUL) || m < 1 || n < 1 || k < 1 ||
+      !dtype_ok(out_dtype) || !x_rows || !w_rows)
+    return fail(INL_E_INVALID, "gemm_bf16_tile: bad arguments");
+  int dev = 0, cus = 0;
+  INL_HIP_TRY(hipGetDevice(&dev));
+  INL_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const int epi = mode == INL_GATE_GEGLU ? EPI_GEGLU : mode == INL_GATE_GELU_MUL ? EPI_GELU_MUL : EPI_PLAIN;
+  static const int32_t tiles[4][2] = {{GemmShapeOf<0>::BM, GemmShapeOf<0>::BN}, {GemmShapeOf<1>::BM, GemmShapeOf<1>::BN},
+                                      {GemmShapeOf<2>::BM, GemmShapeOf<2>::BN}, {GemmShapeOf<3>::BM, GemmShapeOf<3>::BN}};
+  const int sh = pick_shape(epi, m, n, k, out_dtype == INL_BF16, cus);
+  *x_rows = tiles[sh][0];
+  *w_rows = tiles[sh][1];
+  return INL_OK;
+}

@@ -49,8 +49,8 @@ def test_gemm_against_fp32(m, n, k, out, cuda, inl):
 def test_gemm_strides_alpha_beta(n, cuda, inl):
     """Strided x, w and y rows (q/k/v-style slices of wider rows), alpha, and
     beta = 1 accumulation into f32 and into bf16 outputs; columns of y outside
-    [0, n) are left untouched. n = 200 is one n-tile (the 128-row kernel
-    shape), n = 512 two (the 256-row shape)."""
+    [0, n) are left untouched. Both sizes run on 64 x 64 tiles; the other
+    tile shapes' accumulating epilogues are in test_tile_shapes."""
     import torch
     m, k = 700, 256
     xs = _rand(torch, cuda, (m, k + 72), 3)
@@ -192,11 +192,11 @@ def test_gated_gemm_config3_full_size(mode, cuda, inl):
 
 
 # Every kernel shape and epilogue: row counts that the cost rule sends to the
-# 64 x 64, 128 x 128, 256 x 128 and 256 x 256 tiles, each with ragged last
-# tiles in m and n. Against f64 products of the same bf16 values, the bound of
+# 64 x 64, 128 x 128, 256 x 128 (the last two sizes) and 256 x 256 tiles, each
+# with ragged last tiles in m and n (test_tile_shapes names each size's tile). Against f64 products of the same bf16 values, the bound of
 # the tests above (bf16 rounding of the output, 1e-5 of the largest |y|).
 SHAPE_CASES = [(1, 40, 32), (63, 72, 96), (65, 136, 768), (1000, 1160, 768), (2500, 1160, 768), (5000, 776, 768),
-               (5000, 1288, 768), (9999, 776, 256), (9000, 1288, 768), (20001, 264, 256)]
+               (5000, 1288, 768), (9999, 776, 256), (9000, 1288, 768), (20001, 264, 256), (5001, 1288, 64), (3000, 1160, 64)]
 
 
 @pytest.mark.parametrize("epi", ["plain", "geglu", "gelu_mul"])
@@ -229,3 +229,51 @@ def test_every_kernel_shape(m, n, k, epi, cuda, inl):
         err = (y.double() - ref).abs()
         bound = 1e-5 * ref.abs().max() + (ref.abs() * 2 ** -8 if od == torch.bfloat16 else 0)
         assert (err <= bound).all(), f"{od}: max error {err.max().item():.3g}"
+
+
+# Each tile shape (rows of x, rows of w) with each epilogue, named so that a new
+# cost rule cannot drop one unseen: ragged last tiles in m and n, rows of x, w
+# and y inside wider ones. The bounds of the tests above.
+PLAIN_TILES = {(64, 64): (70, 40, 64), (128, 128): (3000, 1160, 64), (128, 256): (5001, 1288, 64),
+               (256, 256): (10001, 1288, 256)}
+GEGLU_TILES = {(64, 64): (70, 40, 64), (128, 128): (1500, 1160, 64), (128, 256): (3000, 1160, 64),
+               (256, 256): (5001, 1288, 256)}
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("epi", ["plain", "accumulate", "geglu", "gelu_mul"])
+@pytest.mark.parametrize("tile", sorted(PLAIN_TILES), ids=lambda t: f"{t[0]}x{t[1]}")
+def test_tile_shapes(tile, epi, out, cuda, inl):
+    import torch
+    m, n, k = (GEGLU_TILES if epi == "geglu" else PLAIN_TILES)[tile]
+    od = torch.float32 if out == "f32" else torch.bfloat16
+    mode = epi if epi in ("geglu", "gelu_mul") else None
+    assert inl.gemm_bf16_tile(m, n, k, od, mode) == tile
+    rows = 2 * n if epi == "geglu" else n
+    x = _rand(torch, cuda, (m, k + 24), m)[:, 8:8 + k]
+    w = _rand(torch, cuda, (rows, k + 16), n, k ** -0.5)[:, :k]
+    mul = _rand(torch, cuda, (m, n + 8), k)[:, :n]
+    gelu = lambda t: torch.nn.functional.gelu(t, approximate="tanh")
+    print(f"case=tile_shapes {tile} {epi} {out} {m}x{n}x{k}", flush=True)
+    base = _rand(torch, cuda, (m + 1, n + 24), 3).to(od)
+    if epi != "accumulate":
+        base[:] = float("nan")
+    buf = base.clone()
+    y = buf[:m, 16:16 + n]
+    p = x.double() @ w.double().T
+    if epi == "accumulate":
+        ref = base[:m, 16:16 + n].double() + 0.5 * p
+        inl.gemm_bf16(x, w, out=y, alpha=0.5, beta=1.0)
+    elif epi == "plain":
+        ref = p
+        inl.gemm_bf16(x, w, out=y)
+    else:
+        ref = gelu(p[:, :n]) * p[:, n:] if epi == "geglu" else gelu(p) * mul.double()
+        inl.gemm_bf16_gated(x, w, epi, mul=mul if epi == "gelu_mul" else None, out=y)
+    torch.cuda.synchronize()
+    err = (y.double() - ref).abs()
+    assert (err <= 1e-5 * ref.abs().max() + (ref.abs() * 2 ** -8 if out == "bf16" else 0)).all(), err.max().item()
+    outside = torch.ones_like(buf, dtype=torch.bool)
+    outside[:m, 16:16 + n] = False
+    a, b = buf[outside], base[outside]
+    assert ((a == b) | (torch.isnan(a.float()) & torch.isnan(b.float()))).all(), "a value outside y was written"
