@@ -6,7 +6,10 @@ takes, one, two and four query heads per K/V head, and row counts at the edges
 of its 16-row blocks, of its text-length classes (32, 64, 128) and of the path
 itself. Tolerances are those of the general path's own test
 (tests/test_qwen3_e2e_gpu.py): f32 cosine 0.99999 and 2e-4 max-abs, bf16
-cosine 0.999 on the bf16-rounded weights."""
+cosine 0.999 on the bf16-rounded weights; and, a text at a time, relative
+distances at twice what right code shows. f32 4e-6. bf16 1.6e-2, of roundings to
+8 bits in some 20 places of two layers: in the oracle, hiding one key of a text
+of 65 to 128 from the rows after it moves its embedding by 6e-2 or more."""
 import numpy as np
 import pytest
 
@@ -44,10 +47,12 @@ def test_few_rows_against_oracle(shape, lengths, dtype, cuda, inl):
         got = enc.encode(ids, cu.tolist()).cpu().numpy().astype(np.float64)
         ref = oq.encode(w, cfg, ids, cu)
         cos = (got * ref).sum(1) / np.linalg.norm(got, axis=1) / np.linalg.norm(ref, axis=1)
+        rel = (np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)).max()
+        print(f"relative error {rel:.3g}", flush=True)
         if dtype == "f32":
-            assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4
+            assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4 and rel <= 4e-6
         else:
-            assert cos.min() >= 0.999
+            assert cos.min() >= 0.999 and rel <= 1.6e-2
     enc.close()
 
 
@@ -67,7 +72,10 @@ def test_few_rows_need_no_larger_workspace(dtype, rows, cuda, inl):
 
 # f32 batches above 464 rows run on the library's own f32 GEMM: row counts at
 # the edges of its 128-row tiles and of the path, and widths with other part
-# counts. The tolerance of the general path.
+# counts. The tolerance of the general path, and a relative distance of 2.5e-6
+# (two layers of f32 sums: 4e-7 to 6e-7, on hipBLASLt 1.3e-6): weights cut to two
+# of their three bf16 parts move the oracle by 8e-6. (The group1 batch of 513 rows
+# has too few tiles and runs on hipBLASLt.)
 @pytest.mark.parametrize("shape,lengths", [("0.6B", [465]), ("0.6B", [200, 312]), ("0.6B", [300, 200, 140, 1]),
                                            ("group1", [500, 13]), ("group4", [512, 257]), ("group1", [500, 200])])
 def test_f32_gemm_rows_against_oracle(shape, lengths, cuda, inl):
@@ -85,6 +93,9 @@ def test_f32_gemm_rows_against_oracle(shape, lengths, cuda, inl):
     ref = oq.encode(w, cfg, ids, cu)
     cos = (got * ref).sum(1) / np.linalg.norm(got, axis=1) / np.linalg.norm(ref, axis=1)
     assert cos.min() >= 0.99999 and np.abs(got - ref).max() <= 2e-4
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f"relative error {rel:.3g}", flush=True)
+    assert rel <= 2.5e-6
 
 
 # Weights that are slices of a larger buffer, one element off a 16-byte boundary:
