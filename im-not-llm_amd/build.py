@@ -51,6 +51,8 @@ EXTRA = {
 # spill could store that register, or hand it to another value, while the
 # load is still in flight. Their kernels must use no scratch; the build reads
 # the compiler's resource-usage remarks and fails if any of them does.
+# gdn_chunk.hip and gemm_f32.hip load through builtins; they are held to the
+# same for speed, their loops filling the register file to a few registers.
 NO_SCRATCH = {"attn_pp.hip", "attn_pp64.hip", "attn_wide.hip", "gdn_chunk.hip", "gemm.hip", "gemm_f32.hip",
               "splade_decoder.hip"}
 RESOURCE_REMARKS = ["-Rpass-analysis=kernel-resource-usage", "-fno-caret-diagnostics"]
@@ -98,7 +100,7 @@ def check_no_scratch(src_name: str, remarks: str) -> None:
         raise RuntimeError(f"{src_name}: remarks without a ScratchSize for " + ", ".join(unsized))
     users = scratch_users(remarks)
     if users:
-        raise RuntimeError(f"{src_name}: kernels with inline-asm loads use scratch: " + ", ".join(users))
+        raise RuntimeError(f"{src_name}: kernels use scratch: " + ", ".join(users))
 
 
 def check_inflight(src_name: str, listing: str) -> None:

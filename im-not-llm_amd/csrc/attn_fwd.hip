@@ -64,6 +64,7 @@
 #include <vector>
 
 #include "attn_kernels.hpp"
+#include "lanes.hpp"
 
 namespace inl {
 
@@ -82,27 +83,11 @@ __device__ __forceinline__ int vcol(int key4) {
   return (key4 & ~15) | ((key4 & 4) << 1) | ((key4 & 8) >> 1);
 }
 
-// Four f32 values as three bf16 parts each (8 bytes a part).
-__device__ __forceinline__ void split4(const f32x4& x, u32x2 (&o)[3]) {
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    f32x2 r = {x[2 * j], x[2 * j + 1]};
-#pragma unroll
-    for (int n = 0; n < 3; ++n) {
-      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-      o[n][j] = u;
-      if (n < 2) {
-        r[0] -= __builtin_bit_cast(float, u << 16);
-        r[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
-      }
-    }
-  }
-}
 // The MFMA operand of eight, in three parts.
 __device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, bf16x8 (&o)[3]) {
   u32x2 x[3], y[3];
-  split4(a, x);
-  split4(b, y);
+  bf16_parts4(a, x);
+  bf16_parts4(b, y);
 #pragma unroll
   for (int n = 0; n < 3; ++n) o[n] = __builtin_bit_cast(bf16x8, (u32x4){x[n][0], x[n][1], y[n][0], y[n][1]});
 }
@@ -256,7 +241,7 @@ __global__ __launch_bounds__(NW * 64, waves_per_simd(D)) void attn_fwd_kernel(At
         if constexpr (ES == 4) {
           const int j = c >> 2, half = c & 1;
           u32x2 o[3];
-          split4(__builtin_bit_cast(f32x4, kst[i]), o);
+          bf16_parts4(__builtin_bit_cast(f32x4, kst[i]), o);
           char* dst = sK + frag_at((row >> 5) * NKJ + j, row & 31, half, (2 * j + half) & 31) + ((c >> 1) & 1) * 8;
 #pragma unroll
           for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(dst + n * 1024) = o[n];
@@ -306,7 +291,7 @@ __global__ __launch_bounds__(NW * 64, waves_per_simd(D)) void attn_fwd_kernel(At
             u32x2 o[3];
             const f32x4 keys = {__builtin_bit_cast(f32x4, vst[i][0])[e], __builtin_bit_cast(f32x4, vst[i][1])[e],
                                 __builtin_bit_cast(f32x4, vst[i][2])[e], __builtin_bit_cast(f32x4, vst[i][3])[e]};
-            split4(keys, o);
+            bf16_parts4(keys, o);
             char* dst = sV + frag_at((db * NKB + kb) * 2 + step, dd & 31, half, db & 3) + h * 8;
 #pragma unroll
             for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(dst + n * 1024) = o[n];

@@ -59,32 +59,16 @@ constexpr int gc_len() { return sizeof(T) == 2 ? 64 : 32; }   // f32: three part
 template <typename T>
 constexpr int gc_parts() { return sizeof(T) == 2 ? 1 : 3; }
 
-// Sum over the four lanes that share lane & 15, in all of them.
-__device__ __forceinline__ float gc_rows4(float x) {
-  float a = x, b = x;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  a = b = a + b;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  return a + b;
-}
-
-// x as N bf16 parts (N = 3: their sum is x to f32's last bit), two values per
-// conversion.
+// An operand's values as N bf16 parts.
 template <int N>
 __device__ __forceinline__ void gc_split(const float (&x)[8], bf16x8 (&p)[N]) {
   u32x4 w[N];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    f32x2 r = {x[2 * j], x[2 * j + 1]};
+    uint32_t u[N];
+    bf16_parts<N>((f32x2){x[2 * j], x[2 * j + 1]}, u);
 #pragma unroll
-    for (int n = 0; n < N; ++n) {
-      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-      w[n][j] = u;
-      if (n + 1 < N) {
-        r[0] -= __builtin_bit_cast(float, u << 16);
-        r[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
-      }
-    }
+    for (int n = 0; n < N; ++n) w[n][j] = u[n];
   }
 #pragma unroll
   for (int n = 0; n < N; ++n) p[n] = __builtin_bit_cast(bf16x8, w[n]);
@@ -230,7 +214,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnChunkParams p) {
       ss += x[s].squares();
       x[s].parts(f[s]);
     }
-    return gc_rows4(ss);
+    return rows4_sum(ss);
   };
   auto dot = [&](const bf16x8 (&a)[4][NP], const bf16x8 (&b)[4][NP]) __attribute__((always_inline)) {
     f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
@@ -487,7 +471,7 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
       float ss = 0.f;
 #pragma unroll
       for (int b = 0; b < 4; ++b) ss += r[b].squares();
-      const float inv = 1.0f / sqrtf(gc_rows4(ss) + 1e-6f);
+      const float inv = 1.0f / sqrtf(rows4_sum(ss) + 1e-6f);
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
@@ -499,7 +483,7 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
       for (int b = 0; b < 8; ++b)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[r] = __builtin_fmaf(S[b][r], x[b][r], s[r]);
-      return gc_rows4((s[0] + s[1]) + (s[2] + s[3]));
+      return rows4_sum((s[0] + s[1]) + (s[2] + s[3]));
     };
     load_row(kr, k_off, 0);
     load_row(qr, q_off, 0);
@@ -585,19 +569,12 @@ __global__ __launch_bounds__(64 * GC_WAVES) void gdn_chunk_rule(GdnChunkParams p
         const int t = 2 * (RT * wave + f) + (ln >> 5), c = ln & 15;   // row, chunk of 4 columns of T or P
         const int ts = c >> 3, hh = (c >> 2) & 1, grp = c & 3;
         if (TS == 1 && ts) continue;   // f32 chunks have 32 columns
-        f32x2 r0 = {rl[f][0], rl[f][1]}, r1 = {rl[f][2], rl[f][3]};
+        u32x2 o[3];
+        bf16_parts4(rl[f], o);
         char* at = smem + ((ln & 16) ? L::PF : L::TF) + ((t >> 4) * TS + ts) * 3 * 1024 +
                    gc_slot(grp, t & 15, x_l(grp, ts)) + 8 * hh;
 #pragma unroll
-        for (int n = 0; n < 3; ++n) {
-          const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r0, bf16x2));
-          const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r1, bf16x2));
-          *reinterpret_cast<u32x2*>(at + n * 1024) = (u32x2){u, w};
-          r0[0] -= __builtin_bit_cast(float, u << 16);
-          r0[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
-          r1[0] -= __builtin_bit_cast(float, w << 16);
-          r1[1] -= __builtin_bit_cast(float, w & 0xffff0000u);
-        }
+        for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(at + n * 1024) = o[n];
       }
       if (wave == GC_WAVES - 1) {
         if (lane < C) {

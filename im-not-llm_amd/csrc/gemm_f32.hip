@@ -131,19 +131,7 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
     for (int i = 0; i < GF_LOADS; ++i) {
       u32x2 o[3];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x2 r = {raw[i][2 * j], raw[i][2 * j + 1]};
-#pragma unroll
-        for (int n = 0; n < 3; ++n) {
-          const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-          o[n][j] = u;
-          if (n < 2) {
-            r[0] -= __builtin_bit_cast(float, u << 16);
-            r[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
-          }
-        }
-      }
+      bf16_parts4(raw[i], o);
 #pragma unroll
       for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(smem + buf * GF_STAGE + dst[i] + n * GF_FRAG) = o[n];
     }

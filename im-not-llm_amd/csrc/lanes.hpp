@@ -1,6 +1,6 @@
-// Cross-lane sums and moves on the VALU (DPP and v_permlane*_swap) for the
-// element-wise kernels, in place of LDS-routed shuffles. Every helper reads
-// other lanes, so it must run with every lane of the wave active.
+// Cross-lane sums and moves on the VALU (DPP and v_permlane*_swap), in place of
+// LDS-routed shuffles: every helper that reads other lanes must run with every
+// lane of the wave active. And the split of f32 values into bf16 parts.
 #pragma once
 
 #include "inl_common.hpp"
@@ -39,5 +39,40 @@ __device__ __forceinline__ float group_sum(float x) {
 }
 
 __device__ __forceinline__ float wave_sum(float x) { return group_sum<64>(x); }
+
+// Sum over the four lanes that share lane & 15, in all of them.
+__device__ __forceinline__ float rows4_sum(float x) {
+  float a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  a = b = a + b;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return a + b;
+}
+
+// Two f32 values as N bf16 parts each, rounded to nearest (u[n]: part n of both,
+// the first in the low half). N = 3: the parts add up to the value, 8 + 8 + 8
+// significand bits, from 2^-110 up to 3.39e38; above, and for infinities, the
+// lower parts are inf - inf.
+template <int N>
+__device__ __forceinline__ void bf16_parts(f32x2 r, uint32_t (&u)[N]) {
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    u[n] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+    if (n + 1 < N) {
+      r[0] -= __builtin_bit_cast(float, u[n] << 16);
+      r[1] -= __builtin_bit_cast(float, u[n] & 0xffff0000u);
+    }
+  }
+}
+// Four values: part n of all is o[n], in order.
+__device__ __forceinline__ void bf16_parts4(const f32x4& x, u32x2 (&o)[3]) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    uint32_t u[3];
+    bf16_parts<3>((f32x2){x[2 * j], x[2 * j + 1]}, u);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) o[n][j] = u[n];
+  }
+}
 
 }  // namespace inl

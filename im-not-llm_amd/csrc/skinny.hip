@@ -154,14 +154,7 @@ __device__ __forceinline__ void store4(char* p, const f32x4& v) {
   }
 }
 
-// Sum over the four lanes that share lane & 15, in all of them.
-__device__ __forceinline__ float rows4_sum(float x) {
-  float a = x, b = x;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  a = b = a + b;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  return a + b;
-}
+// Maximum over the four lanes that share lane & 15, in all of them.
 __device__ __forceinline__ float rows4_max(float x) {
   float a = x, b = x;
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
