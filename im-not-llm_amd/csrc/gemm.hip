@@ -447,25 +447,27 @@ int gemm_launch_shape(GemmParams p, int epi, bool bf, bool acc, int64_t m, int64
   return INL_OK;
 }
 
-// The shape with the least estimated time: q tiles one after another on the
-// fullest CU, each kst stages of `stage` us and `drain` us of epilogue (halved
-// for bf16 outputs: it is the time of the stores). Fitted to the seven
-// EmbeddingGemma projections at 1 to 60,000 rows (k 256 to 1,152, n 256 to
-// 2,304): us per GEMM of the shapes 0 / 1 / 2 / 3
-//   768 -> 768 f32:   1 row 18.1 / 13.7 / 9.8 / 6.9,   2,500 20.1 / 15.7 / 11.4 / 10.3,
-//                     10,000 23.4 / 22.5 / 22.7 / 28.4, 60,000 91 / 101 / 115 / 184
-//   GEGLU 768 -> 1,152: 1,000 rows 20.0 / 15.2 / 11.3 / 14.1, 5,000 25.1 / 27.0 / 28.8 / 42.1
-//   256 -> 768 f32:   21,658 rows 28.9 / 22.3 / 20.5 / 27.0
-// Before, all outputs wider than 256 ran on shape 0 and the others on shape 1.
-int pick_shape(int epi, int64_t m, int64_t n, int64_t k, bool bf, int cus) {
+// The shape with the least estimated time: `start` us until the first tile is
+// under way, then q tiles one after another on the fullest CU, each kst stages of
+// `stage` us and `drain` us of epilogue. Fitted to the seven EmbeddingGemma
+// projections (k 256 to 1,152, n 256 to 2,304) and the MLP of the 0.6B shape at
+// 500 to 139,124 rows, so that no size is slower by more than 3 % than on shape 0
+// (n up to 256: shape 1), which all outputs took before there were four. us per
+// GEMM of the shapes 0 / 1 / 2 / 3
+//   768 -> 768 f32:     1,000 rows 19.2 / 14.6 / 10.3 / 8.0, 6,000 22.0 / 18.7 / 17.4 / 19.8,
+//                       10,000 23.8 / 22.7 / 21.6 / 29.7, 64,000 94 / 109 / 132 / 214
+//   GEGLU 768 -> 1,152: 2,000 rows 20.8 / 16.5 / 16.5 / 19.8, 8,000 44.6 / 44.7 / 40.9 / 62.6
+//   256 -> 768 f32:     3,000 rows 11.7 / 9.6 / 7.3 / 7.9, 12,000 14.9 / 15.4 / 15.6 / 15.9,
+//                       48,000 49.2 / 41.6 / 35.6 / 51.7
+int pick_shape(int epi, int64_t m, int64_t n, int64_t k, int cus) {
   struct Cost {
-    int bn, bm, wpc;
-    float stage, drain, alone;   // alone: us per stage of a tile that has its CU to itself
+    int bn, bm;
+    float stage, drain, start;
   };
-  static const Cost costs[4] = {{GemmShapeOf<0>::BN, GemmShapeOf<0>::BM, 1, 0.55f, 13.f, 0.55f},
-                                {GemmShapeOf<1>::BN, GemmShapeOf<1>::BM, 2, 0.58f, 4.5f, 0.58f},
-                                {GemmShapeOf<2>::BN, GemmShapeOf<2>::BM, 2, 0.28f, 2.4f, 0.28f},
-                                {GemmShapeOf<3>::BN, GemmShapeOf<3>::BM, 2, 0.106f, 0.6f, 0.157f}};
+  static const Cost costs[4] = {{GemmShapeOf<0>::BN, GemmShapeOf<0>::BM, 0.56f, 11.f, 0.f},
+                                {GemmShapeOf<1>::BN, GemmShapeOf<1>::BM, 0.51f, 3.2f, 4.4f},
+                                {GemmShapeOf<2>::BN, GemmShapeOf<2>::BM, 0.25f, 2.2f, 2.9f},
+                                {GemmShapeOf<3>::BN, GemmShapeOf<3>::BM, 0.13f, 0.48f, 3.7f}};
   const float kst = (float)(k / GM_BK);
   int best = 0;
   float least = 0.f;
@@ -473,8 +475,7 @@ int pick_shape(int epi, int64_t m, int64_t n, int64_t k, bool bf, int cus) {
     const Cost& c = costs[i];
     const int64_t bno = epi == EPI_GEGLU ? c.bn / 2 : c.bn;
     const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + bno - 1) / bno);
-    const float q = (float)((tiles + cus - 1) / cus), rounds = (float)((tiles + (int64_t)cus * c.wpc - 1) / ((int64_t)cus * c.wpc));
-    const float t = std::max(rounds * kst * c.alone, q * (kst * c.stage + (bf ? 0.53f : 1.f) * c.drain));
+    const float t = c.start + (float)((tiles + cus - 1) / cus) * (kst * c.stage + c.drain);
     if (i == 0 || t < least) {
       least = t;
       best = i;
@@ -523,7 +524,7 @@ int gemm_launch(int epi, int64_t m, int64_t n, int64_t k, const void* x, int64_t
   p.alpha = alpha;
   p.beta = beta;
   const bool bf = out_dtype == INL_BF16, acc = beta != 0.f;
-  const int sh = pick_shape(epi, m, n, k, bf, cus);
+  const int sh = pick_shape(epi, m, n, k, cus);
   switch (sh) {
     case 0: return gemm_launch_shape<0>(p, epi, bf, acc, m, k, cus, stream);
     case 1: return gemm_launch_shape<1>(p, epi, bf, acc, m, k, cus, stream);
@@ -554,11 +555,10 @@ extern "C" int inl_gemm_bf16_gated_fwd(int64_t m, int64_t n, int64_t k, const vo
                      mul_stride, out_dtype, y, y_stride, 1.f, 0.f, stream);
 }
 
-extern "C" int inl_gemm_bf16_tile(int32_t mode, int64_t m, int64_t n, int64_t k, int32_t out_dtype, int32_t* x_rows,
-                                  int32_t* w_rows) {
+extern "C" int inl_gemm_bf16_tile(int32_t mode, int64_t m, int64_t n, int64_t k, int32_t* x_rows, int32_t* w_rows) {
   using namespace inl;
   if ((mode != 0 && mode != INL_GATE_GEGLU && mode != INL_GATE_GELU_MUL) || m < 1 || n < 1 || k < 1 ||
-      !dtype_ok(out_dtype) || !x_rows || !w_rows)
+      !x_rows || !w_rows)
     return fail(INL_E_INVALID, "gemm_bf16_tile: bad arguments");
   int dev = 0, cus = 0;
   INL_HIP_TRY(hipGetDevice(&dev));
@@ -566,7 +566,7 @@ extern "C" int inl_gemm_bf16_tile(int32_t mode, int64_t m, int64_t n, int64_t k,
   const int epi = mode == INL_GATE_GEGLU ? EPI_GEGLU : mode == INL_GATE_GELU_MUL ? EPI_GELU_MUL : EPI_PLAIN;
   static const int32_t tiles[4][2] = {{GemmShapeOf<0>::BM, GemmShapeOf<0>::BN}, {GemmShapeOf<1>::BM, GemmShapeOf<1>::BN},
                                       {GemmShapeOf<2>::BM, GemmShapeOf<2>::BN}, {GemmShapeOf<3>::BM, GemmShapeOf<3>::BN}};
-  const int sh = pick_shape(epi, m, n, k, out_dtype == INL_BF16, cus);
+  const int sh = pick_shape(epi, m, n, k, cus);
   *x_rows = tiles[sh][0];
   *w_rows = tiles[sh][1];
   return INL_OK;

@@ -555,7 +555,7 @@ _gemm = _sig("inl_gemm_bf16_fwd", ctypes.c_int, c_i64, c_i64, c_i64, c_void_p, c
              c_void_p, c_i64, ctypes.c_float, ctypes.c_float, c_void_p)
 _gemm_gated = _sig("inl_gemm_bf16_gated_fwd", ctypes.c_int, c_i64, c_i64, c_i64, c_void_p, c_i64, c_void_p, c_i64,
                    c_i32, c_void_p, c_i64, c_i32, c_void_p, c_i64, c_void_p)
-_gemm_tile = _sig("inl_gemm_bf16_tile", ctypes.c_int, c_i32, c_i64, c_i64, c_i64, c_i32, ctypes.POINTER(c_i32),
+_gemm_tile = _sig("inl_gemm_bf16_tile", ctypes.c_int, c_i32, c_i64, c_i64, c_i64, ctypes.POINTER(c_i32),
                   ctypes.POINTER(c_i32))
 INL_GATE_GEGLU, INL_GATE_GELU_MUL = 1, 2
 _embed = _sig("inl_embed_fwd", ctypes.c_int, c_i64, c_void_p, c_void_p, c_i64, c_i32, c_i32, c_void_p, c_i64,
@@ -673,14 +673,13 @@ def gemm_bf16_gated(x, w, mode, *, mul=None, out=None, out_dtype=None, stream=No
     return out
 
 
-def gemm_bf16_tile(m, n, k, out_dtype, mode=None):
+def gemm_bf16_tile(m, n, k, mode=None):
     """``inl_gemm_bf16_tile``: (rows of x, rows of w) per tile of the kernel
     that ``gemm_bf16`` (``mode=None``) or ``gemm_bf16_gated`` launches for a
     shape."""
-    import torch
     a, b = c_i32(), c_i32()
     code = {None: 0, "geglu": INL_GATE_GEGLU, "gelu_mul": INL_GATE_GELU_MUL}[mode]
-    _check(_gemm_tile(code, m, n, k, 0 if out_dtype == torch.float32 else 1, ctypes.byref(a), ctypes.byref(b)))
+    _check(_gemm_tile(code, m, n, k, ctypes.byref(a), ctypes.byref(b)))
     return a.value, b.value
 
 

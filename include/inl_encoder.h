@@ -89,7 +89,7 @@ int inl_gemm_bf16_gated_fwd(int64_t m, int64_t n, int64_t k, const void* x,
 /* The tile (rows of x, rows of w) that a call of this shape takes on the
  * current device; mode 0 is inl_gemm_bf16_fwd. For tests and traces. */
 int inl_gemm_bf16_tile(int32_t mode, int64_t m, int64_t n, int64_t k,
-                       int32_t out_dtype, int32_t* x_rows, int32_t* w_rows);
+                       int32_t* x_rows, int32_t* w_rows);
 
 /* out[t, :] = f32(table[ids[t], :]): the token embedding (candle Embedding,
  * qwen3/mod.rs:322-323,350) into an f32 residual stream. ids are device
